@@ -97,19 +97,19 @@ _Static_assert(sizeof(k_quant_job) == 32, "k_quant_job must match quant_job in i
 
 /*
  * A batch of GEMVs as launches: one list-quantiser launch for the distinct
- * activations of streaming jobs that carry f32 x, one slab launch, one
- * streaming launch. Device tables, in this order: quant list, jobs, slab
- * workgroup descriptors, streaming workgroup descriptors.
+ * activations of streaming jobs that carry f32 x, one slab launch, one wide
+ * launch, one streaming launch. Device tables, in this order: quant list,
+ * jobs, slab workgroup descriptors, streaming ones, wide ones.
  */
 struct sllm_gfx950_plan {
     void      *tables_dev;
     void      *scratch_dev;    /* q / act of streaming jobs that quantise without giving buffers */
     uint32_t   n_quant;
     uint32_t   n_jobs;
-    uint32_t   slab_wg;        /* multiple of 8 (empty descriptors pad it) */
+    uint32_t   slab_wg, wide_wg;   /* multiples of 8 (empty descriptors pad them) */
     uint32_t   st_wg, st_lds, st_threads;
     int        st_lpr_idx;
-    uint64_t   slab_target;    /* bytes of packed weights per slab */
+    uint64_t   slab_target, wide_target;   /* bytes of packed weights per slab */
 };
 
 static struct {
@@ -120,7 +120,7 @@ static struct {
     char           name[520];
     hipModule_t    mod, dec_mod;
     hipFunction_t  k_quant, k_quant_list, k_quant_host, k_host_done;
-    hipFunction_t  k_slab;
+    hipFunction_t  k_slab, k_wide;
     hipFunction_t  k_stream[N_LPR];
     hipFunction_t  k_copy;
     hipFunction_t  k_gemm[15];
@@ -166,7 +166,7 @@ static pthread_mutex_t g_noalloc_mtx = PTHREAD_MUTEX_INITIALIZER;
 static struct {
     k_quant_job quant[SLLM_GFX950_NOALLOC_MAX_JOBS];
     k_gemv_job  jobs[SLLM_GFX950_NOALLOC_MAX_JOBS];
-    uint8_t     is_slab[SLLM_GFX950_NOALLOC_MAX_JOBS];
+    uint8_t     path[SLLM_GFX950_NOALLOC_MAX_JOBS];
     uint8_t     tables[SLLM_GFX950_NOALLOC_SCRATCH_BYTES];
 } g_noalloc;
 
@@ -234,6 +234,7 @@ static int load_functions(void) {
     HIP_TRY(hipModuleGetFunction(&g.k_copy, g.mod, "sllm_k_copy"));
     HIP_TRY(hipModuleGetFunction(&g.k_checksum, g.mod, "sllm_k_checksum"));
     HIP_TRY(hipModuleGetFunction(&g.k_slab, g.mod, "sllm_k_gemv_slab"));
+    HIP_TRY(hipModuleGetFunction(&g.k_wide, g.mod, "sllm_k_gemv_wide"));
     HIP_TRY(hipModuleGetFunction(&g.k_gemm[0], g.mod, "sllm_k_gemm_mfma_s1x1"));
     HIP_TRY(hipModuleGetFunction(&g.k_gemm[1], g.mod, "sllm_k_gemm_mfma_2x2"));
     HIP_TRY(hipModuleGetFunction(&g.k_gemm[2], g.mod, "sllm_k_gemm_mfma_4x2"));
@@ -594,6 +595,11 @@ int sllm_gfx950_quant_act(const float *x, size_t n, size_t n_tok, int8_t *q,
  * (K <= 2560), variant 1 16 lanes x 7 chunks (K <= 7168). A job carrying
  * f32 x is quantised inside the kernel: no quantiser launch.
  *
+ * Wide kernel (SLAB_MAX_K < K <= WIDE_MAX_K): the slab kernel's scheme with
+ * sixteen waves, one row per wave and pass, so groups of 16 rows, up to the
+ * K that four chunks a lane cover. One launch where the streaming kernel
+ * takes two; 4096 x 14336 from f32 x: 8.0 us against 22.0.
+ *
  * Streaming kernel (larger K, or forced with path 1): LPR lanes per row, W
  * waves looping over groups of 64/LPR rows inside a slab of rows_per_wg rows,
  * reading a quantised row staged in LDS; jobs carrying f32 x are quantised
@@ -606,6 +612,10 @@ int sllm_gfx950_quant_act(const float *x, size_t n, size_t n_tok, int8_t *q,
 #define SLAB_THREADS     256
 #define SLAB_MAX_K       7168
 #define SLAB_MAX_ROWS    1024
+#define WIDE_THREADS     1024
+#define WIDE_MAX_K       16384
+#define WIDE_GROUP       16u     /* rows per pass: one per wave */
+#define WIDE_KIB         544     /* largest slab of a batch: 136 KiB per four waves, as the slab kernel's */
 #define SLAB_DEFAULT_KIB 136     /* 32 slabs per BitNet-2B FFN matrix: 2-4 % faster than 34 (128 KiB) */
 
 typedef struct slab_geom { int lpr, cpl; } slab_geom;
@@ -634,12 +644,30 @@ static int slab_path(size_t n_rows, size_t k) {
     return (uint64_t) n_rows * (k / 4) + 32 <= 0xFFFF0000u;
 }
 
+/* which kernel a job of this shape takes */
+enum { PATH_STREAM = 0, PATH_SLAB = 1, PATH_WIDE = 2 };
+static int job_path(size_t n_rows, size_t k) {
+    if (slab_path(n_rows, k)) return PATH_SLAB;
+    if (g.force_path != 1 && k > SLAB_MAX_K && k <= WIDE_MAX_K &&
+        (uint64_t) n_rows * (k / 4) + 32 <= 0xFFFF0000u) return PATH_WIDE;
+    return PATH_STREAM;
+}
+
+/* chunks per lane of the wide kernel: 64 lanes of 16-byte chunks per row */
+static uint32_t wide_variant(size_t k) { return (uint32_t) ((k + 4095) / 4096); }
+
 /* Slabs of a job: about `target` bytes of weights each, at least one group
  * each, and few enough groups per slab for its dots to fit in LDS. */
 static uint64_t slab_default_target(void) { return (uint64_t) (g.slab_kib ? g.slab_kib : SLAB_DEFAULT_KIB) * 1024u; }
 
-static uint32_t slab_count(size_t n_rows, size_t k, int variant, uint64_t target) {
-    const uint64_t group = 4u * (uint64_t) (64 / k_slab_geom[variant].lpr);
+static uint64_t slab_default_wide(void) { return (uint64_t) (g.slab_kib ? g.slab_kib : WIDE_KIB) * 1024u; }
+
+/* rows of one pass of a workgroup */
+static uint32_t group_rows(int path, int variant) {
+    return path == PATH_WIDE ? WIDE_GROUP : 4u * (uint32_t) (64 / k_slab_geom[variant].lpr);
+}
+
+static uint32_t slab_count(size_t n_rows, size_t k, uint64_t group, uint64_t target) {
     const uint64_t n_groups = (n_rows + group - 1) / group;
     const uint64_t max_groups = SLAB_MAX_ROWS / group;
     uint64_t slabs = ((uint64_t) n_rows * (k / 4) + target / 2) / target;
@@ -720,7 +748,7 @@ static size_t align256(size_t v) { return (v + 255u) & ~(size_t) 255u; }
 
 /* streaming jobs that quantise x into plan scratch (carry x, no q / act) */
 static int takes_scratch(const sllm_gfx950_gemv_job *j) {
-    return j->x != NULL && j->q == NULL && !slab_path(j->n_rows, j->n);
+    return j->x != NULL && j->q == NULL && job_path(j->n_rows, j->n) == PATH_STREAM;
 }
 
 /* scratch bytes for one quantised row of width k: q, then act */
@@ -740,10 +768,10 @@ static size_t plan_scratch_bytes(const sllm_gfx950_gemv_job *jobs, size_t n_jobs
 }
 
 /* workgroups a job takes (streaming: and the rows each one owns) */
-static uint32_t job_workgroups(const k_gemv_job *kj, int slab, uint32_t *rows, uint64_t target) {
-    if (slab) {
+static uint32_t job_workgroups(const k_gemv_job *kj, int path, uint32_t *rows, uint64_t target) {
+    if (path != PATH_STREAM) {
         *rows = 0;
-        return slab_count(kj->n_rows, kj->k, (int) kj->variant, target);
+        return slab_count(kj->n_rows, kj->k, group_rows(path, (int) kj->variant), target);
     }
     *rows = stream_shape_for().rows_per_wg;
     return (kj->n_rows + *rows - 1) / *rows;
@@ -761,18 +789,20 @@ static uint64_t pad8(uint64_t v) { return (v + 7u) & ~(uint64_t) 7u; }
  * by plan_descriptors.
  */
 static int plan_layout(const sllm_gfx950_gemv_job *jobs, size_t n_jobs, sllm_gfx950_plan *p,
-                       k_quant_job *kq, k_gemv_job *kj, uint8_t *is_slab) {
+                       k_quant_job *kq, k_gemv_job *kj, uint8_t *path) {
     const stream_shape ss = stream_shape_for();
-    uint64_t slab_wg = 0, st_wg = 0;
+    uint64_t slab_wg = 0, st_wg = 0, wide_wg = 0;
     size_t st_lds = 0, scratch_at = 0;
     p->n_quant = 0;
     for (size_t i = 0; i < n_jobs; ++i) {
         k_gemv_job *j = &kj[i];
         int st = job_to_kernel(&jobs[i], i, j);
         if (st != SLLM_GFX950_OK) return st;
-        is_slab[i] = (uint8_t) slab_path(j->n_rows, j->k);
-        if (is_slab[i]) {
+        path[i] = (uint8_t) job_path(j->n_rows, j->k);
+        if (path[i] == PATH_SLAB) {
             j->variant = (uint32_t) slab_variant_for(j->k);
+        } else if (path[i] == PATH_WIDE) {
+            j->variant = wide_variant(j->k);
         } else if (j->x != NULL) {
             const int scratch = j->q == NULL;
             uint32_t e = 0;
@@ -798,21 +828,29 @@ static int plan_layout(const sllm_gfx950_gemv_job *jobs, size_t n_jobs, sllm_gfx
     }
     /* Slabs of the default size fill the chip with a batch of 35 MB and up;
      * a smaller batch (one FFN set, 13 MB) gets slabs sized so that its
-     * workgroups still cover every CU once. */
-    uint64_t slab_bytes = 0;
+     * workgroups still cover every CU once. The same for the wide jobs. */
+    uint64_t slab_bytes = 0, wide_bytes = 0;
     for (size_t i = 0; i < n_jobs; ++i) {
-        if (is_slab[i]) slab_bytes += (uint64_t) kj[i].n_rows * (kj[i].k / 4);
+        const uint64_t bytes = (uint64_t) kj[i].n_rows * (kj[i].k / 4);
+        if (path[i] == PATH_SLAB) slab_bytes += bytes;
+        if (path[i] == PATH_WIDE) wide_bytes += bytes;
     }
     p->slab_target = slab_default_target();
+    p->wide_target = slab_default_wide();
     if (g.slab_kib == 0 && slab_bytes > 0 && slab_bytes < p->slab_target * (uint64_t) g.cu) {
         p->slab_target = (slab_bytes + (uint64_t) g.cu - 1) / (uint64_t) g.cu;
+    }
+    if (g.slab_kib == 0 && wide_bytes > 0 && wide_bytes < p->wide_target * (uint64_t) g.cu) {
+        p->wide_target = (wide_bytes + (uint64_t) g.cu - 1) / (uint64_t) g.cu;
     }
     for (size_t i = 0; i < n_jobs; ++i) {
         k_gemv_job *j = &kj[i];
         uint32_t rows;
-        const uint64_t wg = job_workgroups(j, is_slab[i], &rows, p->slab_target);
-        if (is_slab[i]) {
+        const uint64_t wg = job_workgroups(j, path[i], &rows, path[i] == PATH_WIDE ? p->wide_target : p->slab_target);
+        if (path[i] == PATH_SLAB) {
             slab_wg += wg;
+        } else if (path[i] == PATH_WIDE) {
+            wide_wg += wg;
         } else {
             st_wg += wg;
             if (j->k > st_lds) st_lds = j->k;
@@ -820,27 +858,32 @@ static int plan_layout(const sllm_gfx950_gemv_job *jobs, size_t n_jobs, sllm_gfx
     }
     slab_wg = pad8(slab_wg);
     st_wg = pad8(st_wg);
-    if (slab_wg > INT32_MAX || st_wg > INT32_MAX) return fail(SLLM_GFX950_ERR_TOO_LARGE, "batch: too many workgroups");
+    wide_wg = pad8(wide_wg);
+    if (slab_wg > INT32_MAX || st_wg > INT32_MAX || wide_wg > INT32_MAX) return fail(SLLM_GFX950_ERR_TOO_LARGE, "batch: too many workgroups");
     p->n_jobs = (uint32_t) n_jobs;
     p->slab_wg = (uint32_t) slab_wg;
     p->st_wg = (uint32_t) st_wg;
+    p->wide_wg = (uint32_t) wide_wg;
     p->st_lds = (uint32_t) st_lds;
     p->st_threads = (uint32_t) (64 * ss.waves);
     p->st_lpr_idx = ss.lpr_idx;
     return SLLM_GFX950_OK;
 }
 
-/* One descriptor per workgroup: slab jobs into sd, streaming jobs into td,
- * each in job order and padded with empty descriptors. */
-static void plan_descriptors(const sllm_gfx950_plan *p, const k_gemv_job *kj, const uint8_t *is_slab,
-                             k_wg_desc *sd, k_wg_desc *td) {
-    uint32_t ns = 0, nt = 0;
+/* One descriptor per workgroup: slab jobs, then streaming jobs, then wide
+ * jobs, each in job order and padded with empty descriptors. */
+static void plan_descriptors(const sllm_gfx950_plan *p, const k_gemv_job *kj, const uint8_t *path, k_wg_desc *d) {
+    k_wg_desc *sd = d, *td = d + p->slab_wg, *wd = td + p->st_wg;
+    uint32_t ns = 0, nt = 0, nw = 0;
     for (uint32_t i = 0; i < p->n_jobs; ++i) {
         uint32_t rows;
-        const uint32_t wg = job_workgroups(&kj[i], is_slab[i], &rows, p->slab_target);
+        const uint32_t wg = job_workgroups(&kj[i], path[i], &rows,
+                                           path[i] == PATH_WIDE ? p->wide_target : p->slab_target);
         for (uint32_t w = 0; w < wg; ++w) {
-            if (is_slab[i]) {
+            if (path[i] == PATH_SLAB) {
                 sd[ns++] = (k_wg_desc) { i, w, wg, w == 0 ? WG_PUBLISH : 0 };
+            } else if (path[i] == PATH_WIDE) {
+                wd[nw++] = (k_wg_desc) { i, w, wg, w == 0 ? WG_PUBLISH : 0 };
             } else {
                 const uint32_t b = w * rows, e = b + rows < kj[i].n_rows ? b + rows : kj[i].n_rows;
                 td[nt++] = (k_wg_desc) { i, b, e, 0 };
@@ -849,6 +892,7 @@ static void plan_descriptors(const sllm_gfx950_plan *p, const k_gemv_job *kj, co
     }
     while (ns < p->slab_wg) sd[ns++] = (k_wg_desc) { 0, 0, 0, 0 };
     while (nt < p->st_wg) td[nt++] = (k_wg_desc) { 0, 0, 0, 0 };
+    while (nw < p->wide_wg) wd[nw++] = (k_wg_desc) { 0, 0, 0, 0 };
 }
 
 static int launch_quant(const float *x, uint32_t n, uint32_t n_tok, int8_t *q, sllm_gfx950_act *act) {
@@ -863,6 +907,7 @@ static int plan_launch(const sllm_gfx950_plan *p, int event) {
     const k_gemv_job *jobs = (const k_gemv_job *) (base + p->n_quant * sizeof(k_quant_job));
     const k_wg_desc *sd = (const k_wg_desc *) (jobs + p->n_jobs);
     const k_wg_desc *td = sd + p->slab_wg;
+    const k_wg_desc *wd = td + p->st_wg;
     k_gemv_job none;
     memset(&none, 0, sizeof none);
     uint32_t zero = 0;
@@ -875,6 +920,11 @@ static int plan_launch(const sllm_gfx950_plan *p, int event) {
         uint32_t n = p->slab_wg;
         void *args[] = { (void *) &jobs, (void *) &sd, &n, &none, &zero };
         st = launch(g.k_slab, p->slab_wg, SLAB_THREADS, 0, args);
+    }
+    if (st == SLLM_GFX950_OK && p->wide_wg) {
+        uint32_t n = p->wide_wg;
+        void *args[] = { (void *) &jobs, (void *) &wd, &n, &none, &zero };
+        st = launch(g.k_wide, p->wide_wg, WIDE_THREADS, 0, args);
     }
     if (st == SLLM_GFX950_OK && p->st_wg) {
         uint32_t n = p->st_wg;
@@ -893,10 +943,10 @@ int sllm_gfx950_plan_create(const sllm_gfx950_gemv_job *jobs, size_t n_jobs,
     sllm_gfx950_plan *p = calloc(1, sizeof *p);
     k_quant_job *kq = malloc(n_jobs * sizeof *kq);
     k_gemv_job *kj = malloc(n_jobs * sizeof *kj);
-    uint8_t *is_slab = malloc(n_jobs);
+    uint8_t *path = malloc(n_jobs);
     uint8_t *host = NULL;
     int st = SLLM_GFX950_OK;
-    if (p == NULL || kq == NULL || kj == NULL || is_slab == NULL) {
+    if (p == NULL || kq == NULL || kj == NULL || path == NULL) {
         st = fail(SLLM_GFX950_ERR_NOMEM, "plan: host tables");
     }
     if (st == SLLM_GFX950_OK) {
@@ -906,18 +956,17 @@ int sllm_gfx950_plan_create(const sllm_gfx950_gemv_job *jobs, size_t n_jobs,
             if (e != hipSuccess) st = hip_fail(e, "plan: activation scratch");
         }
     }
-    if (st == SLLM_GFX950_OK) st = plan_layout(jobs, n_jobs, p, kq, kj, is_slab);
+    if (st == SLLM_GFX950_OK) st = plan_layout(jobs, n_jobs, p, kq, kj, path);
     if (st == SLLM_GFX950_OK) {
         const size_t qbytes = p->n_quant * sizeof *kq, jbytes = n_jobs * sizeof *kj;
-        const size_t dbytes = ((size_t) p->slab_wg + p->st_wg) * sizeof(k_wg_desc);
+        const size_t dbytes = ((size_t) p->slab_wg + p->st_wg + p->wide_wg) * sizeof(k_wg_desc);
         const size_t bytes = qbytes + jbytes + dbytes;
         host = malloc(bytes);
         if (host == NULL) st = fail(SLLM_GFX950_ERR_NOMEM, "plan: table staging");
         if (st == SLLM_GFX950_OK) {
             memcpy(host, kq, qbytes);
             memcpy(host + qbytes, kj, jbytes);
-            k_wg_desc *sd = (k_wg_desc *) (host + qbytes + jbytes);
-            plan_descriptors(p, kj, is_slab, sd, sd + p->slab_wg);
+            plan_descriptors(p, kj, path, (k_wg_desc *) (host + qbytes + jbytes));
             hipError_t e = hipMalloc(&p->tables_dev, bytes);
             if (e == hipSuccess) e = hipMemcpy(p->tables_dev, host, bytes, hipMemcpyHostToDevice);
             if (e != hipSuccess) st = hip_fail(e, "plan: job tables");
@@ -926,7 +975,7 @@ int sllm_gfx950_plan_create(const sllm_gfx950_gemv_job *jobs, size_t n_jobs,
     free(host);
     free(kq);
     free(kj);
-    free(is_slab);
+    free(path);
     if (st != SLLM_GFX950_OK) {
         if (p) {
             if (p->tables_dev) hipFree(p->tables_dev);
@@ -1006,10 +1055,10 @@ int sllm_gfx950_gemv_batch_noalloc(const sllm_gfx950_gemv_job *jobs, size_t n_jo
     sllm_gfx950_plan p;
     memset(&p, 0, sizeof p);
     p.scratch_dev = g.noalloc_dev;
-    int st = plan_layout(jobs, n_jobs, &p, g_noalloc.quant, g_noalloc.jobs, g_noalloc.is_slab);
+    int st = plan_layout(jobs, n_jobs, &p, g_noalloc.quant, g_noalloc.jobs, g_noalloc.path);
     if (st == SLLM_GFX950_OK) {
         const size_t qbytes = p.n_quant * sizeof(k_quant_job), jbytes = n_jobs * sizeof(k_gemv_job);
-        const size_t dbytes = ((size_t) p.slab_wg + p.st_wg) * sizeof(k_wg_desc);
+        const size_t dbytes = ((size_t) p.slab_wg + p.st_wg + p.wide_wg) * sizeof(k_wg_desc);
         const size_t bytes = qbytes + jbytes + dbytes;
         if (rows + bytes > cap) {
             st = fail(SLLM_GFX950_ERR_TOO_LARGE, "gemv_batch_noalloc: %zu bytes of rows and tables, the array holds %zu",
@@ -1018,8 +1067,7 @@ int sllm_gfx950_gemv_batch_noalloc(const sllm_gfx950_gemv_job *jobs, size_t n_jo
             uint8_t *host = g_noalloc.tables;
             memcpy(host, g_noalloc.quant, qbytes);
             memcpy(host + qbytes, g_noalloc.jobs, jbytes);
-            k_wg_desc *sd = (k_wg_desc *) (host + qbytes + jbytes);
-            plan_descriptors(&p, g_noalloc.jobs, g_noalloc.is_slab, sd, sd + p.slab_wg);
+            plan_descriptors(&p, g_noalloc.jobs, g_noalloc.path, (k_wg_desc *) (host + qbytes + jbytes));
             p.tables_dev = (uint8_t *) g.noalloc_dev + rows;
             hipError_t e = hipMemcpyAsync(p.tables_dev, host, bytes, hipMemcpyHostToDevice, g.stream);
             if (e != hipSuccess) st = hip_fail(e, "gemv_batch_noalloc: tables");
@@ -1044,21 +1092,23 @@ static int single_launch(const sllm_gfx950_gemv_job *j) {
     const k_gemv_job *no_jobs = NULL;
     const k_wg_desc *no_descs = NULL;
     uint32_t zero = 0;
-    if (slab_path(kj.n_rows, kj.k)) {
-        kj.variant = (uint32_t) slab_variant_for(kj.k);
+    const int path = job_path(kj.n_rows, kj.k);
+    if (path != PATH_STREAM) {
+        const int wide = path == PATH_WIDE;
+        kj.variant = wide ? wide_variant(kj.k) : (uint32_t) slab_variant_for(kj.k);
         uint32_t rows, flags = 0;
-        uint32_t wg = job_workgroups(&kj, 1, &rows, slab_default_target());
+        uint32_t wg = job_workgroups(&kj, path, &rows, wide ? slab_default_wide() : slab_default_target());
         if (g.slab_kib == 0) {
             /* The slab size targets batches, whose many jobs fill the chip;
              * a launch of its own spreads over one group of rows per
              * workgroup, up to one workgroup per CU. */
-            const uint32_t group = 4u * (uint32_t) (64 / k_slab_geom[kj.variant].lpr);
+            const uint32_t group = group_rows(path, (int) kj.variant);
             const uint32_t n_groups = (kj.n_rows + group - 1) / group;
             const uint32_t want = n_groups < (uint32_t) g.cu ? n_groups : (uint32_t) g.cu;
             if (wg < want) wg = want;
         }
         void *args[] = { (void *) &no_jobs, (void *) &no_descs, &zero, &kj, &flags };
-        return launch(g.k_slab, wg, SLAB_THREADS, 0, args);
+        return launch(wide ? g.k_wide : g.k_slab, wg, wide ? WIDE_THREADS : SLAB_THREADS, 0, args);
     }
     if (kj.x != NULL) {
         if (kj.q == NULL) {

@@ -132,7 +132,8 @@ __device__ __forceinline__ int wave_sum(int v) {
 // must be active: callers keep the reduction out of divergent code.
 template <int LPR>
 __device__ __forceinline__ int group_sum(int v) {
-    static_assert(LPR == 4 || LPR == 8 || LPR == 16, "lanes per row");
+    static_assert(LPR == 4 || LPR == 8 || LPR == 16 || LPR == 64, "lanes per row");
+    if (LPR == 64) return wave_sum(v);
     v += __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, false);    // quad_perm [1,0,3,2]
     v += __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, false);    // quad_perm [2,3,0,1]
     if (LPR >= 8) v += __builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, false);  // row_half_mirror
@@ -296,13 +297,13 @@ struct gemv_job {
     int32_t       *out_i;      // raw int32 dots, or null
     uint32_t       n_rows;     // N
     uint32_t       k;          // K, a multiple of 128
-    uint32_t       variant;    // slab kernel geometry: 0 = (8 lanes, 5 chunks), 1 = (16, 7)
+    uint32_t       variant;    // slab geometry: 0 = (8 lanes, 5 chunks), 1 = (16, 7); wide: chunks per lane
     uint32_t       pad;
 };
 
 // One workgroup's share of a batch, in job `job`:
-//   slab kernel      slab a of b slabs of the job (b == 0: padding); flags
-//                    WG_PUBLISH
+//   slab and wide    slab a of b slabs of the job (b == 0: padding); flags
+//   kernels          WG_PUBLISH
 //   streaming kernel rows [a, b) (a >= b: padding)
 // Empty descriptors pad the table to a multiple of 8 workgroups.
 struct wg_desc {
@@ -360,13 +361,19 @@ constexpr uint32_t SLAB_MAX_ROWS = 1024;
 
 static_assert(8 * 5 * 64 <= SLAB_MAX_K && 16 * 7 * 64 <= SLAB_MAX_K, "slab geometries read inside the LDS row");
 
-struct slab_shared {
-    int8_t  q[SLAB_MAX_K];
-    int32_t dots[SLAB_MAX_ROWS];
-    float   red_f[SLAB_WAVES];
-    int     red_i[SLAB_WAVES];
-    int     red_a[SLAB_WAVES];
+// Up to MAXK elements of a row and the dots of MAX_ROWS rows in LDS, TH
+// threads
+template <int TH, uint32_t MAXK, uint32_t MAX_ROWS>
+struct slab_lds {
+    static constexpr int THREADS = TH, WAVES = TH / 64;
+    static constexpr uint32_t MAX_K = MAXK;
+    int8_t  q[MAXK];
+    int32_t dots[MAX_ROWS];
+    float   red_f[WAVES];
+    int     red_i[WAVES];
+    int     red_a[WAVES];
 };
+typedef slab_lds<SLAB_THREADS, SLAB_MAX_K, SLAB_MAX_ROWS> slab_shared;
 
 // Every load of the slab kernel is unconditional: a skipped load (a branch
 // around it, or an exec-masked block the wave jumps over when no lane needs

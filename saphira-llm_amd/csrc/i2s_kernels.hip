@@ -34,9 +34,13 @@ namespace {
 // the workgroup's four waves; slab a of b takes the a-th run of consecutive
 // groups. (Dealing the groups round-robin instead, so that a job's slabs
 // sweep it side by side, measured no faster.)
-template <int LPR, int CPL, int XV, int QV, bool QUANT>
+template <int LPR, int CPL, int XV, int QV, bool QUANT, typename SH>
 __device__ __forceinline__ void slab_block(const gemv_job &job, uint32_t slab, uint32_t n_slabs,
-                                           uint32_t flags, slab_shared &S) {
+                                           uint32_t flags, SH &S) {
+    constexpr int SLAB_THREADS = SH::THREADS, SLAB_WAVES = SH::WAVES;
+    constexpr uint32_t SLAB_MAX_K = SH::MAX_K;
+    static_assert(LPR * CPL * 64 <= (int) SLAB_MAX_K && 4 * XV * SLAB_THREADS >= LPR * CPL * 64 &&
+                  16 * QV * SLAB_THREADS >= LPR * CPL * 64, "the dots read inside the LDS row, all of it written");
     constexpr uint32_t RPW = 64 / LPR;
     constexpr uint32_t G = SLAB_WAVES * RPW;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -207,6 +211,21 @@ __device__ __forceinline__ void slab_block(const gemv_job &job, uint32_t slab, u
         }
     }
 }
+
+// ---------------------------------------------------------------------------
+// wide GEMV (7168 < K <= 16384): the slab block with sixteen waves and a wave
+// per row, CPL 16-byte chunks a lane (K <= 4096 CPL). One row group is then
+// 16 rows, so that a lone tensor of 4096 rows still covers every CU, and all
+// of its weights are in flight before the activation is quantised: the launch
+// is bound by that prologue's memory latency, and by HBM where a workgroup
+// has many groups. 4096 x 14336 from f32 x (14.7 MB): 8.0 us a call, 1.85
+// TB/s, against 22.0 us for a one-workgroup quantiser launch and the
+// streaming kernel.
+// ---------------------------------------------------------------------------
+
+constexpr int WIDE_THREADS = 1024;
+constexpr uint32_t WIDE_MAX_K = 16384, WIDE_MAX_ROWS = 1024;
+typedef slab_lds<WIDE_THREADS, WIDE_MAX_K, WIDE_MAX_ROWS> wide_shared;
 
 // ---------------------------------------------------------------------------
 // streaming GEMV (any K up to the LDS limit): waves loop over row groups with
@@ -1629,6 +1648,40 @@ sllm_k_gemv_slab(const gemv_job *__restrict__ jobs, const wg_desc *__restrict__ 
     } else {                                                                     // K <= 7168
         if (quant) slab_block<16, 7, 7, 2, true>(job, slab, n_slabs, flags, S);
         else slab_block<16, 7, 7, 2, false>(job, slab, n_slabs, flags, S);
+    }
+}
+
+// Wide GEMV: blocks of WIDE_THREADS; descriptors and the single-job form as
+// sllm_k_gemv_slab's. job.variant: chunks per lane (2, 3 or 4).
+extern "C" __global__ void __launch_bounds__(WIDE_THREADS)
+sllm_k_gemv_wide(const gemv_job *__restrict__ jobs, const wg_desc *__restrict__ descs,
+                 uint32_t n_wg, gemv_job single, uint32_t single_flags) {
+    __shared__ wide_shared S;
+    gemv_job job;
+    uint32_t slab, n_slabs, flags;
+    if (descs != nullptr) {
+        const wg_desc d = descs[xcd_slot(n_wg)];
+        if (d.b == 0) return;
+        job = jobs[d.job];
+        slab = d.a;
+        n_slabs = d.b;
+        flags = d.flags;
+    } else {
+        job = single;
+        slab = blockIdx.x;
+        n_slabs = gridDim.x;
+        flags = (single_flags & ~WG_PUBLISH) | (blockIdx.x == 0 ? WG_PUBLISH : 0u);
+    }
+    const bool quant = job.x != nullptr;
+    if (job.variant == 2) {                                                      // K <= 8192
+        if (quant) slab_block<64, 2, 2, 1, true>(job, slab, n_slabs, flags, S);
+        else slab_block<64, 2, 2, 1, false>(job, slab, n_slabs, flags, S);
+    } else if (job.variant == 3) {                                               // K <= 12288
+        if (quant) slab_block<64, 3, 3, 1, true>(job, slab, n_slabs, flags, S);
+        else slab_block<64, 3, 3, 1, false>(job, slab, n_slabs, flags, S);
+    } else {                                                                     // K <= 16384
+        if (quant) slab_block<64, 4, 4, 1, true>(job, slab, n_slabs, flags, S);
+        else slab_block<64, 4, 4, 1, false>(job, slab, n_slabs, flags, S);
     }
 }
 
