@@ -124,6 +124,7 @@ static struct {
     hipFunction_t  k_stream[N_LPR];
     hipFunction_t  k_copy;
     hipFunction_t  k_gemm[15];
+    hipFunction_t  k_gemm_tail[15];      /* dk4x4, dk2x2, dq1x1, dq2x1 (their k_gemm index) for K % 256 == 128 */
     hipFunction_t  k_gemm_t[5];
     hipFunction_t  k_gemm_s;             /* plans of a few tokens as one stream per workgroup */
     hipFunction_t  k_gemm_rope[2];       /* dk2x2, dk4x4 with the chunk's cache store */
@@ -250,6 +251,10 @@ static int load_functions(void) {
     HIP_TRY(hipModuleGetFunction(&g.k_gemm[12], g.mod, "sllm_k_gemm_dk2x2"));
     HIP_TRY(hipModuleGetFunction(&g.k_gemm[13], g.mod, "sllm_k_gemm_dq1x1"));
     HIP_TRY(hipModuleGetFunction(&g.k_gemm[14], g.mod, "sllm_k_gemm_dq2x1"));
+    HIP_TRY(hipModuleGetFunction(&g.k_gemm_tail[9], g.mod, "sllm_k_gemm_dk4x4_tail"));
+    HIP_TRY(hipModuleGetFunction(&g.k_gemm_tail[12], g.mod, "sllm_k_gemm_dk2x2_tail"));
+    HIP_TRY(hipModuleGetFunction(&g.k_gemm_tail[13], g.mod, "sllm_k_gemm_dq1x1_tail"));
+    HIP_TRY(hipModuleGetFunction(&g.k_gemm_tail[14], g.mod, "sllm_k_gemm_dq2x1_tail"));
     HIP_TRY(hipModuleGetFunction(&g.k_gemm_rope[0], g.mod, "sllm_k_gemm_dk2x2_rope"));
     HIP_TRY(hipModuleGetFunction(&g.k_gemm_rope[1], g.mod, "sllm_k_gemm_dk4x4_rope"));
     HIP_TRY(hipModuleGetFunction(&g.k_gemm_glu[0], g.mod, "sllm_k_gemm_dk2x2_glu"));
@@ -1163,7 +1168,7 @@ _Static_assert(sizeof(k_gemm_args) == 128, "k_gemm_args must match gemm_args in 
  * waves instead of spreading them along the rows; shapes 3 and 4 stage their
  * tile through LDS -- 3 with two buffers, one workgroup per CU; 4 with one,
  * two per CU; shapes 5..8 copy it straight into an LDS ring). Shapes 3 and
- * up need K % 256 == 0. */
+ * up need K % 256 == 0; 9, 12, 13 and 14 have a form for K % 256 == 128. */
 #define N_GEMM_TILES 15
 #define GEMM_DL_FIRST 5
 static const uint32_t k_gemm_tokens[N_GEMM_TILES] = { 16, 32, 64, 128, 128, 16, 32, 32, 64, 64, 64, 32, 32, 16, 32 };
@@ -1203,24 +1208,24 @@ static int gemm_prepare(const sllm_gfx950_gemm_job *jobs, size_t n_jobs, size_t 
         if ((uint64_t) m * jobs[j].n_rows > (uint64_t) 1 << 40) return fail(SLLM_GFX950_ERR_TOO_LARGE, "gemm: m x rows too large");
     }
     int tile = g.force_gemm_tile - 1;
-    if (tile < 0 && n % 256 == 0) {
+    if (tile < 0) {
         /* measured on MI355X (K = 2560 and 6912, 4 to 512 tokens): the
          * direct-load tiles win everywhere. Up to 64 tokens the sixteen-wave
          * 16 x 64 / 32 x 64 tiles (four K groups; each tensor streamed once
          * per token tile); to 256 tokens the eight-wave 32 x 128, or 32 x 64
          * when that grid would cover under half the CUs; above 256 tokens the
          * eight-wave 64 x 256 when its grid covers three quarters of the
-         * CUs, else 32 x 128. */
+         * CUs, else 32 x 128. K % 256 == 128 takes the same shapes with a
+         * half last super-step (gemm_function). */
         const uint64_t cu = (uint64_t) (g.cu > 0 ? g.cu : 256);
         if (m <= 16) tile = 13;
         else if (m <= 64) tile = gemm_grid(14, jobs, n_jobs, m) * 4 >= cu * 3 ? 14 : 13;
         else if (m <= 256) tile = gemm_grid(12, jobs, n_jobs, m) * 2 >= cu ? 12 : 14;
         else tile = gemm_grid(9, jobs, n_jobs, m) * 4 >= cu * 3 ? 9 : 12;
-    } else if (tile < 0) {
-        /* K % 256 != 0: split-K tiles up to 64 tokens, else 64 x 128 */
-        tile = m <= 64 ? 0 : 2;
+        if (n % 256 != 0 && tile == 12 && m > (size_t) 65535 * 32) tile = 2;   /* past its grid: the 64-token tile */
+    } else if (tile >= 3 && n % 256 != 0) {
+        tile = 2;
     }
-    if (tile >= 3 && n % 256 != 0) tile = 2;
     const uint32_t rows_per_wg = k_gemm_rows[tile], tok_per_wg = k_gemm_tokens[tile];
     memset(a, 0, sizeof *a);
     uint64_t gx = 0;
@@ -1242,6 +1247,12 @@ static int gemm_prepare(const sllm_gfx950_gemm_job *jobs, size_t n_jobs, size_t 
     return SLLM_GFX950_OK;
 }
 
+/* the kernel of a chosen tile: the shapes gemm_prepare picks by itself have a
+ * form for K % 256 == 128, and no other shape of theirs is picked for it */
+static hipFunction_t gemm_function(int tile, size_t n) {
+    return n % 256 != 0 && g.k_gemm_tail[tile] != NULL ? g.k_gemm_tail[tile] : g.k_gemm[tile];
+}
+
 int sllm_gfx950_gemm_multi(const sllm_gfx950_gemm_job *jobs, size_t n_jobs, size_t n, const int8_t *q,
                            const sllm_gfx950_act *act, size_t m) {
     NEED_OPEN();
@@ -1251,7 +1262,7 @@ int sllm_gfx950_gemm_multi(const sllm_gfx950_gemm_job *jobs, size_t n_jobs, size
     const int st = gemm_prepare(jobs, n_jobs, n, q, act, m, &a, &tile, &gx, &gy);
     if (st != SLLM_GFX950_OK || gx == 0) return st;
     void *args[] = { &a };
-    HIP_TRY(hipModuleLaunchKernel(g.k_gemm[tile], (uint32_t) gx, (uint32_t) gy, 1, k_gemm_threads[tile], 1, 1, 0,
+    HIP_TRY(hipModuleLaunchKernel(gemm_function(tile, n), (uint32_t) gx, (uint32_t) gy, 1, k_gemm_threads[tile], 1, 1, 0,
                                   g.stream, args, NULL));
     return SLLM_GFX950_OK;
 }
@@ -1264,7 +1275,7 @@ int sllm_shim_gemm_qkv_rope(const sllm_gfx950_gemm_job jobs[3], size_t n, const 
     uint64_t gx, gy;
     const int st = gemm_prepare(jobs, 3, n, q, act, m, &a, &tile, &gx, &gy);
     if (st != SLLM_GFX950_OK || gx == 0) return st;
-    const int which = tile == 12 ? 0 : (tile == 9 ? 1 : -1);
+    const int which = n % 256 != 0 ? -1 : (tile == 12 ? 0 : (tile == 9 ? 1 : -1));
     if (which < 0 || r->hd == 0 || k_gemm_rows[tile] % r->hd != 0 || r->half == 0 || r->half % 4 != 0 ||
         2 * r->half > r->hd || r->hd % 8 != 0)
         return SLLM_SHIM_NOT_FUSED;
@@ -1287,7 +1298,7 @@ int sllm_shim_gemm_glu(const uint8_t *w_gate, const uint8_t *w_up, size_t n_rows
     uint64_t gx, gy;
     const int st = gemm_prepare(jobs, 2, n, q, act, m, &a, &tile, &gx, &gy);
     if (st != SLLM_GFX950_OK || gx == 0) return st;
-    const int which = tile == 12 ? 0 : (tile == 9 ? 1 : -1);
+    const int which = n % 256 != 0 ? -1 : (tile == 12 ? 0 : (tile == 9 ? 1 : -1));
     if (which < 0) return SLLM_SHIM_NOT_FUSED;
     /* one tile per BN / 2 rows of each tensor: the same grid as the pair */
     const uint32_t half_rows = k_gemm_rows[tile] / 2;
@@ -1310,7 +1321,7 @@ int sllm_shim_gemm_res(const uint8_t *w, size_t n_rows, size_t n, const int8_t *
     uint64_t gx, gy;
     const int st = gemm_prepare(&job, 1, n, q, act, m, &a, &tile, &gx, &gy);
     if (st != SLLM_GFX950_OK || gx == 0) return st;
-    const int which = tile == 12 ? 0 : (tile == 9 ? 1 : (tile == 13 ? 2 : (tile == 14 ? 3 : -1)));
+    const int which = n % 256 != 0 ? -1 : tile == 12 ? 0 : (tile == 9 ? 1 : (tile == 13 ? 2 : (tile == 14 ? 3 : -1)));
     if (which < 0) return SLLM_SHIM_NOT_FUSED;
     void *args[] = { &a, (void *) &res };
     HIP_TRY(hipModuleLaunchKernel(g.k_gemm_res[which], (uint32_t) gx, (uint32_t) gy, 1, k_gemm_threads[tile], 1, 1, 0,

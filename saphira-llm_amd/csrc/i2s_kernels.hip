@@ -920,7 +920,10 @@ __device__ __forceinline__ void gemm_tile_epilogue(uint8_t *S, const gemm_view &
 // GLU: a gate + up tile (V.w gate, V.w2 up, n_rows each): BN / 2 rows of
 // each tensor, gate's in K group 0's half of the weight slot and up's in
 // group 1's, so that the epilogue finds both factors of every output.
-template <int TM, int TN, int STAGES, int KG = 1, bool ROPE = false, bool GLU = false, bool RES = false>
+// TAIL: K % 256 == 128. The last super-step has one I2_S block: the copies of
+// its second half fetch the first half's granules and chunks again, and the
+// lane groups that would take them (g >= 2) multiply codes of zero.
+template <int TM, int TN, int STAGES, int KG = 1, bool ROPE = false, bool GLU = false, bool RES = false, bool TAIL = false>
 __device__ __forceinline__ void gemm_dl_tile(const gemm_view &V, uint32_t k, uint32_t m, uint32_t by,
                                              const gemm_rope *R = nullptr) {
     constexpr uint32_t BM = 16u * TM, BN = 64u * TN;
@@ -948,8 +951,9 @@ __device__ __forceinline__ void gemm_dl_tile(const gemm_view &V, uint32_t k, uin
     const uint32_t wave = wave_all & 3u, kgrp = wave_all >> 2;   // place in the tile, K group
     const uint32_t g = lane >> 4, li = lane & 15u;
     static_assert(!GLU || KG == 2, "a gate + up tile is two K groups, one per tensor");
+    static_assert(!TAIL || WL, "a half super-step needs the chunk-wise weight copies");
     const uint32_t t0 = by * BM, n0 = V.tile * (GLU ? BN / 2u : BN);
-    const uint32_t nsup = k / 256u, kb = k >> 2;
+    const uint32_t nsup = TAIL ? k / 256u + 1u : k / 256u, kb = k >> 2;
     // the epilogue's operands, loaded now so that their latency hides behind
     // the main loop: w_scale, and token t0 + tid's act for the first BM threads
     float ep_ws = 0.0f, ep_ws2 = 0.0f;
@@ -968,11 +972,13 @@ __device__ __forceinline__ void gemm_dl_tile(const gemm_view &V, uint32_t k, uin
     // copy sources: instruction j of this wave fills LDS granules
     // (4 j + wave) * 64 + lane of the token and the weight block
     const int8_t *asrc[TM];
+    uint32_t aback[TM];                             // TAIL: back into the block there is, at the last super-step
 #pragma unroll
     for (int j = 0; j < TM; ++j) {
         const uint32_t p = ((uint32_t) j * 4u + wave) * 64u + lane;
         const uint32_t t = p >> 4, gr = (p & 15u) ^ (t & 15u);
         asrc[j] = V.q + (size_t) min(t0 + t, m - 1) * k + gr * 16u;
+        aback[j] = gr >= 8u ? 128u : 0u;
     }
     const uint8_t *bsrc[TN];
     uint32_t bch[TN];                               // WL: the chunk (of CR) each copy lane fetches
@@ -1000,14 +1006,15 @@ __device__ __forceinline__ void gemm_dl_tile(const gemm_view &V, uint32_t k, uin
         uint8_t *base = S + (s % STAGES) * (WL ? A_BYTES : STAGE);
 #pragma unroll
         for (int j = 0; j < TM; ++j)
-            __builtin_amdgcn_global_load_lds((const void *) (asrc[j] + sc * 256u),
+            __builtin_amdgcn_global_load_lds((const void *) (asrc[j] + sc * 256u - (TAIL && sc == nsup - 1 ? aback[j] : 0u)),
                                              LDS_PTR(base + ((uint32_t) j * 4u + wave) * 1024u), 16, 0, 0);
         if (WL) {
             const uint32_t it = min(s / KG, iters - 1);
             uint8_t *wbase = S + A_REGION + ((s / KG) % D) * WSLOT + kgrp * (BN / KG) * PB;
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
-                const uint32_t ch = KG * it + bch[j] / 4u < nsup ? bch[j] : (bch[j] & 3u);
+                uint32_t ch = KG * it + bch[j] / 4u < nsup ? bch[j] : (bch[j] & 3u);
+                if (TAIL && KG * it + ch / 4u == nsup - 1) ch &= ~2u;
                 __builtin_amdgcn_global_load_lds((const void *) (bsrc[j] + it * PB + ch * 16u),
                                                  LDS_PTR(wbase + ((uint32_t) j * 4u + wave) * 1024u), 16, 0, 0);
             }
@@ -1054,6 +1061,10 @@ __device__ __forceinline__ void gemm_dl_tile(const gemm_view &V, uint32_t k, uin
         u32x4 raw[TN];
 #pragma unroll
         for (int tn = 0; tn < TN; ++tn) raw[tn] = *reinterpret_cast<const u32x4 *>(sw + boff + (uint32_t) tn * BROW16);
+        if (TAIL && s == nsup - 1 && g >= 2u) {
+#pragma unroll
+            for (int tn = 0; tn < TN; ++tn) raw[tn] = (u32x4) { 0, 0, 0, 0 };
+        }
         i32x4v a[2][TM], b[2][TN];
 #pragma unroll
         for (int tm = 0; tm < TM; ++tm) a[0][tm] = *reinterpret_cast<const i32x4v *>(st + aoff[0] + (uint32_t) tm * 4096u);
@@ -1100,11 +1111,11 @@ __device__ __forceinline__ void gemm_dl_tile(const gemm_view &V, uint32_t k, uin
 }
 
 // the tile of a three-job launch (gemm_args) or of a plan (gemm_table)
-template <int TM, int TN, int STAGES, int KG = 1, bool ROPE = false>
+template <int TM, int TN, int STAGES, int KG = 1, bool ROPE = false, bool TAIL = false>
 __device__ __forceinline__ void gemm_dl_block(const gemm_args &G, const gemm_rope *R = nullptr) {
     uint32_t bx, by;
     gemm_place(bx, by);
-    gemm_dl_tile<TM, TN, STAGES, KG, ROPE>(gemm_pick(G, bx), G.k, G.m, by, R);
+    gemm_dl_tile<TM, TN, STAGES, KG, ROPE, false, false, TAIL>(gemm_pick(G, bx), G.k, G.m, by, R);
 }
 
 // a gate + up launch: job 0 of gemm_args is gate, job 1 up (the same
@@ -1760,6 +1771,20 @@ extern "C" __global__ void __launch_bounds__(1024)
 sllm_k_gemm_dq1x1(gemm_args G) { gemm_dl_block<1, 1, 16, 4>(G); }
 extern "C" __global__ void __launch_bounds__(1024)
 sllm_k_gemm_dq2x1(gemm_args G) { gemm_dl_block<2, 1, 12, 4>(G); }
+
+// K % 256 == 128: the shapes the host picks by itself, with a half last
+// super-step. Against the tiles that load their operands straight into
+// registers, which these K had to themselves before, quantiser included:
+// 77 tokens x 1000 rows x 1408 23.2 -> 7.8 us (of it about 4.4 in two
+// launches), a larger one 409 -> 137 us.
+extern "C" __global__ void __launch_bounds__(512)
+sllm_k_gemm_dk4x4_tail(gemm_args G) { gemm_dl_block<4, 4, 4, 2, false, true>(G); }
+extern "C" __global__ void __launch_bounds__(512)
+sllm_k_gemm_dk2x2_tail(gemm_args G) { gemm_dl_block<2, 2, 4, 2, false, true>(G); }
+extern "C" __global__ void __launch_bounds__(1024)
+sllm_k_gemm_dq1x1_tail(gemm_args G) { gemm_dl_block<1, 1, 16, 4, false, true>(G); }
+extern "C" __global__ void __launch_bounds__(1024)
+sllm_k_gemm_dq2x1_tail(gemm_args G) { gemm_dl_block<2, 1, 12, 4, false, true>(G); }
 
 // the same tiles over a plan's table of tensors
 extern "C" __global__ void __launch_bounds__(256)
