@@ -127,7 +127,8 @@ enum { IN_PLAIN = 0, IN_RESID = 1, IN_EMBED = 2, IN_SILU = 3 };
 #define LM_WG_PER_CU 2    /* output workgroups per CU (LDS: 32 KiB each); 2 ran 4 us per token faster than 4 */
 #define CHK_THREADS  512
 #define CLM_THREADS  256
-#define CLM_TOK      4    /* tokens per chunk output-head workgroup */
+#define CLM_TOK      16   /* tokens and rows per chunk output-head workgroup */
+#define CLM_ROWS     64
 #define CS_TOK       8    /* tokens per chunk scores workgroup (half that up to CS_SMALL tokens) */
 #define CS_SMALL     128
 #define CSW_THREADS  1024 /* the one-wave-unit scores kernel: sixteen waves per CU */
@@ -1072,7 +1073,7 @@ static int launch_chunk(sllm_gfx950_ctx *c, int32_t n, int32_t base, int all_log
         /* l_out, output_norm per token, every token's row of logits */
         st = prep(c, n, IN_RESID, B->proj, B->fi, NULL, m->output_norm, (uint32_t) e, 0, B->xn);
         const uint32_t n_tb = (uint32_t) ((n + CLM_TOK - 1) / CLM_TOK);
-        const uint32_t n_rb = (uint32_t) ((m->n_vocab + CLM_THREADS - 1) / CLM_THREADS);
+        const uint32_t n_rb = (uint32_t) ((m->n_vocab + CLM_ROWS - 1) / CLM_ROWS);
         k_chk_lm L = { B->xn, m->tok_embd, B->logits, (uint32_t) e, (uint32_t) m->n_vocab, (uint32_t) n,
                        pad8(n_tb * n_rb) };
         void *largs[] = { &L };

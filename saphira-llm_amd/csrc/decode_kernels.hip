@@ -1446,8 +1446,19 @@ struct chk_lm {
 };
 static_assert(sizeof(chk_lm) == 40, "chk_lm must match decode.c");
 
-constexpr int CLM_THREADS = 256;        // one row per lane
-constexpr int CLM_TOK = 4;              // tokens per workgroup
+constexpr int CLM_THREADS = 256;        // four waves, side by side along the rows
+constexpr uint32_t CLM_TOK = 16;        // tokens per workgroup
+constexpr uint32_t CLM_ROWS = 16 * (CLM_THREADS / 64);
+constexpr uint32_t CLM_RING = 3;        // pairs of 32-element steps in LDS per wave
+constexpr uint32_t CLM_W = 16 * 128, CLM_SLOT = CLM_W + 4 * 1024;   // a pair's embedding rows, then its tokens
+
+// Where the output head reads element i (a multiple of 4) of token t's
+// normalised row of k: tiles of 16 tokens, then steps of 32 elements, each
+// two blocks of 64 lanes x four floats -- lane 16 b + t % 16 of block h holds
+// elements 8 b + 4 h .. + 3 of the step.
+__device__ __forceinline__ size_t clm_at(uint32_t t, uint32_t i, uint32_t k) {
+    return (((size_t) (t / CLM_TOK) * (k / 32) + i / 32) * 2 + (i / 4) % 2) * 256 + ((i % 32) / 8 * 16 + t % CLM_TOK) * 4;
+}
 
 } // namespace
 
@@ -1516,7 +1527,7 @@ __device__ __forceinline__ void chk_prep_body(const chk_prep &P, float *xs, doub
                 m = fmaxf(m, fabsf(v[c]));
             }
             *reinterpret_cast<f32x4 *>(xs + i) = v;
-            if (P.xn_out != nullptr) *G_CAST(f32x4, P.xn_out + row + i) = v;
+            if (P.xn_out != nullptr) *G_CAST(f32x4, P.xn_out + clm_at(t, i, k)) = v;
         }
     }
     if (P.q_out == nullptr) return;                  // uniform
@@ -1616,78 +1627,116 @@ sllm_k_chk_kv_store(dec_attn A) {
     }
 }
 
-// The output head over a chunk. Lane = one row; a workgroup takes 256 rows
-// for CLM_TOK tokens. Each row . xn[t] is formed as src/ops.c:106-154 orders
-// it: accumulator 8j + l collects element 32i + 8j + l by FMA over i; then
-// (acc_0 + acc_2) + (acc_1 + acc_3) per l, t_l = a_l + a_{l+4},
-// (t0 + t1) + (t2 + t3). The normalised rows are the same for every lane,
-// so they are read as wave-uniform values. Workgroups for the same rows sit
-// next to each other on one XCD, so the rows come from its L2 after the
-// first token block.
-extern "C" __global__ void __launch_bounds__(CLM_THREADS)
+// The output head over a chunk. Each row . xn[t] is formed as
+// src/ops.c:106-154 orders it: accumulator 8j + l collects element 32i + 8j + l
+// by FMA over i; then (acc_0 + acc_2) + (acc_1 + acc_3) per l, t_l = a_l +
+// a_{l+4}, (t0 + t1) + (t2 + t3).
+//
+// One v_mfma_f32_16x16x1_4b is four 16 x 16 outer products, each product added
+// to its accumulator by one correctly rounded FMA (measured: the bits of fmaf
+// for any operands, denormals, infinities and NaN included). Its four blocks
+// take j = 0..3 of one l for 16 rows and 16 tokens, so a step of 32 elements
+// is eight of them, on eight chains; lane 16 j + r holds elements 8j .. 8j + 7
+// of row r and of token r. The chains are as long as the reference's and
+// independent.
+//
+// Each wave has an LDS ring of its own, so nothing is shared and no barrier
+// is needed: global_load_lds copies two steps at a time, the embedding as 8
+// rows x 128 bytes (whole lines; a lane's own 16 bytes of 16 rows would be
+// half lines) with chunk c of row r at slot c ^ (r % 8), the tokens as whole
+// blocks of the layout clm_at.
+//
+// Bound by the FMAs: 256 bytes of operands bring 1024 of them, and with no
+// copies at all 128 tokens x 128256 rows x 2560 take 820 us (two waves per
+// SIMD). This takes 1000 us, 512 tokens 3.8 ms, 16 tokens 155 us (657 MB,
+// 4.2 TB/s); one row per lane and the tokens through the scalar unit took 2.69
+// and 9.7 ms. Measured slower here: the operands straight into registers
+// (1050 us with 16 rows a wave, 1220 with 32), rings of four and six pairs at
+// one workgroup per CU (1340). Workgroups for the same rows and different
+// tokens sit next to each other on one XCD, so the rows come from its L2 after
+// the first.
+extern "C" __global__ void __launch_bounds__(CLM_THREADS, 2)
 sllm_k_chk_lm_head(chk_lm L) {
+    typedef float f32x16 __attribute__((ext_vector_type(16)));
+    __shared__ __attribute__((aligned(1024))) uint8_t S[CLM_THREADS / 64 * CLM_RING * CLM_SLOT];
     const uint32_t n_tb = (L.n_tok + CLM_TOK - 1) / CLM_TOK;
     const uint32_t b = xcd_slot(L.n_wg);
     const uint32_t tb = b % n_tb, rb = b / n_tb;
-    const uint32_t e = L.n_embd, steps = e / 32;
-    if (rb * CLM_THREADS >= L.n_vocab) return;
-    const uint32_t row = min(rb * CLM_THREADS + threadIdx.x, L.n_vocab - 1);
-    const uint32_t t0 = tb * CLM_TOK;
-    const GLOBAL u32x4 *w = G_CAST(const u32x4, L.embd + (size_t) row * e);
-    // the normalised rows do not change during the launch: constant
-    // address space, so the wave-uniform reads are scalar loads
-    typedef __attribute__((address_space(4))) const float cfloat;
-    cfloat *xb[CLM_TOK];
+    const uint32_t e = L.n_embd, pairs = e / 64, lane = threadIdx.x & 63;      // n_embd % 128 == 0
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t row0 = rb * CLM_ROWS + wave * 16;
+    if (row0 >= L.n_vocab) return;                 // a whole wave; no barriers below
+    uint8_t *ring = S + wave * CLM_RING * CLM_SLOT;
+    const uint8_t *wsrc[2];                        // copy j: rows 8 j + lane / 8
 #pragma unroll
-    for (int u = 0; u < CLM_TOK; ++u) xb[u] = (cfloat *) (L.xn + (size_t) min(t0 + (uint32_t) u, L.n_tok - 1) * e);
-    float acc[CLM_TOK][32];
-#pragma unroll
-    for (int u = 0; u < CLM_TOK; ++u) {
-#pragma unroll
-        for (int j = 0; j < 32; ++j) acc[u][j] = 0.0f;
+    for (uint32_t j = 0; j < 2; ++j) {
+        const uint32_t r = 8 * j + lane / 8;
+        wsrc[j] = (const uint8_t *) (L.embd + (size_t) min(row0 + r, L.n_vocab - 1) * e) + ((lane % 8) ^ (r % 8)) * 16;
     }
-    // 32 elements (64 bytes) of the row per step; steps alternate between
-    // two buffers so that the next step's loads are in flight during this one
-    auto load = [&](uint32_t i, u32x4 (&h)[4]) {
-        const uint32_t at = 4 * min(i, steps - 1);
+    const float *xsrc = L.xn + (size_t) tb * CLM_TOK * e + lane * 4;
+    f32x16 acc[8];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) h[c] = w[at + (uint32_t) c];
+    for (int l = 0; l < 8; ++l) acc[l] = (f32x16) (0.0f);
+    // pair p into a slot (past the end, the last pair again: never read)
+    auto issue = [&](uint32_t p, uint32_t slot) {
+        const uint32_t pc = min(p, pairs - 1);
+        uint8_t *to = ring + slot * CLM_SLOT;
+#pragma unroll
+        for (uint32_t j = 0; j < 2; ++j)
+            __builtin_amdgcn_global_load_lds((const void *) (wsrc[j] + pc * 128u), LDS_PTR(to + j * 1024u), 16, 0, 0);
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j)
+            __builtin_amdgcn_global_load_lds((const void *) (xsrc + (4 * pc + j) * 256u), LDS_PTR(to + CLM_W + j * 1024u), 16, 0, 0);
     };
-    auto step = [&](uint32_t i, const u32x4 (&h)[4]) {
-        float hf[32];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const f32x8 f = __builtin_convertvector(__builtin_bit_cast(f16x8, h[c]), f32x8);
+    for (uint32_t p = 0; p < CLM_RING - 1; ++p) issue(p, p);
+    const uint32_t r16 = lane % 16, j4 = lane / 16;
+    uint32_t slot = 0;
+    for (uint32_t p = 0; p < pairs; ++p) {
+        wait_vmem<(int) (CLM_RING - 2) * 6>();      // pair p's six copies done
+        __builtin_amdgcn_sched_barrier(0);
+        const uint8_t *at = ring + slot * CLM_SLOT;
+        u32x4 w[2];
+        f32x4 x[4];
 #pragma unroll
-            for (int l = 0; l < 8; ++l) hf[8 * c + l] = f[l];
+        for (uint32_t q = 0; q < 2; ++q) w[q] = *reinterpret_cast<const u32x4 *>(at + r16 * 128 + ((4 * q + j4) ^ (r16 % 8)) * 16);
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) x[q] = *reinterpret_cast<const f32x4 *>(at + CLM_W + q * 1024 + lane * 16);
+        const uint32_t prev = slot == 0 ? CLM_RING - 1 : slot - 1;
+        __builtin_amdgcn_s_waitcnt(0xC07F);         // lgkmcnt(0): the slot before is read out too
+        __builtin_amdgcn_sched_barrier(0);
+        issue(p + CLM_RING - 1, prev);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const f32x8 hf = __builtin_convertvector(__builtin_bit_cast(f16x8, w[q]), f32x8);
+#pragma unroll
+            for (int l = 0; l < 8; ++l)
+                acc[l] = __builtin_amdgcn_mfma_f32_16x16x1f32(hf[l], x[2 * q + l / 4][l % 4], acc[l], 0, 0, 0);
         }
-#pragma unroll
-        for (int u = 0; u < CLM_TOK; ++u) {
-            cfloat *x = xb[u] + 32 * i;
-#pragma unroll
-            for (int j = 0; j < 32; ++j) acc[u][j] = fmaf(hf[j], x[j], acc[u][j]);
-        }
-    };
-    u32x4 ha[4], hb[4];
-    load(0, ha);
-    uint32_t i = 0;
-    for (; i + 1 < steps; i += 2) {
-        load(i + 1, hb);
-        step(i, ha);
-        load(i + 2, ha);
-        step(i + 1, hb);
+        slot = slot + 1 == CLM_RING ? 0 : slot + 1;
     }
-    if (i < steps) step(i, ha);
-    if (rb * CLM_THREADS + threadIdx.x >= L.n_vocab) return;
+    wait_vmem<0>();                                 // no copy may land after the wave leaves
+    const uint32_t t = tb * CLM_TOK + lane % 16;
+    if (t >= L.n_tok) return;
+    // register 4 j + r of an accumulator: row 4 (lane / 16) + r, j
+    f32x4 o;
 #pragma unroll
-    for (int u = 0; u < CLM_TOK; ++u) {
-        if (t0 + (uint32_t) u < L.n_tok) {
-            float a[8];
+    for (int r = 0; r < 4; ++r) {
+        float a[8];
 #pragma unroll
-            for (int l = 0; l < 8; ++l) a[l] = (acc[u][l] + acc[u][16 + l]) + (acc[u][8 + l] + acc[u][24 + l]);
-            const float s0 = a[0] + a[4], s1 = a[1] + a[5], s2 = a[2] + a[6], s3 = a[3] + a[7];
-            L.logits[(size_t) (t0 + (uint32_t) u) * L.n_vocab + row] = (s0 + s1) + (s2 + s3);
-        }
+        for (int l = 0; l < 8; ++l) a[l] = (acc[l][r] + acc[l][8 + r]) + (acc[l][4 + r] + acc[l][12 + r]);
+        const float s0 = a[0] + a[4], s1 = a[1] + a[5], s2 = a[2] + a[6], s3 = a[3] + a[7];
+        o[r] = (s0 + s1) + (s2 + s3);
+    }
+    const uint32_t row = row0 + 4 * j4;
+    GLOBAL float *to = G_CAST(float, L.logits) + (size_t) t * L.n_vocab + row;
+    if (L.n_vocab % 4 == 0 && row < L.n_vocab) {
+        *reinterpret_cast<GLOBAL f32x4 *>(to) = o;
+    } else {
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r)
+            if (row + r < L.n_vocab) to[r] = o[r];
     }
 }
 

@@ -141,6 +141,16 @@ __device__ __forceinline__ int group_sum(int v) {
     return v;
 }
 
+// Copies from global memory straight into LDS (__builtin_amdgcn_global_load_lds)
+// count as vector memory loads: wait until at most N are outstanding.
+template <int N>
+__device__ __forceinline__ void wait_vmem() {   // s_waitcnt vmcnt(N), the other counters untouched
+    static_assert(N >= 0 && N < 64, "vmcnt");
+    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+
+#define LDS_PTR(p) ((__attribute__((address_space(3))) void *) (p))
+
 // ---------------------------------------------------------------------------
 // activation quantiser (src/i2s_gemm.c:45-83)
 // ---------------------------------------------------------------------------

@@ -711,14 +711,6 @@ __device__ __forceinline__ void gemm_lds_block(const gemm_args &G) {
 // step the next step's operand reads and weight unpacking are interleaved
 // with the current step's MFMAs, which keep the matrix unit busy while the
 // SIMD issues them.
-template <int N>
-__device__ __forceinline__ void wait_vmem() {   // s_waitcnt vmcnt(N), the other counters untouched
-    static_assert(N >= 0 && N < 64, "vmcnt");
-    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-
-#define LDS_PTR(p) ((__attribute__((address_space(3))) void *) (p))
-
 // XCD-aware placement. Workgroups are dealt to the eight XCDs round-robin by
 // linear id (x fastest); XCD s is given a contiguous run of the tiles, row
 // tile slowest, so the workgroups that share a weight tile (all its token
