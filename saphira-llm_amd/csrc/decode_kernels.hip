@@ -671,104 +671,85 @@ __device__ __forceinline__ void chk_scores_body(const dec_attn &A, uint32_t n_to
 }
 
 extern "C" __global__ void __launch_bounds__(ATT_THREADS)
-sllm_k_chk_scores(dec_attn A, uint32_t n_tok) { chk_scores_body<8>(A, n_tok); }
-extern "C" __global__ void __launch_bounds__(ATT_THREADS)
 sllm_k_chk_scores4(dec_attn A, uint32_t n_tok) { chk_scores_body<4>(A, n_tok); }
 
-// The chunk's scores as units of one wave: (KV head, query head, 8 tokens,
-// 64 positions), lane r = position s0 + r, the same dot chains as above.
-// The lane streams its key from the cache (L2) in chunks of 32 dimensions
-// (four slices of eight: each load instruction reads 16 bytes of 64
-// consecutive positions, 32 bytes apart, rather than 64 separate rows), the
-// next chunk in flight while this one is used, so the wave needs no LDS and
-// no barrier; the queries come
-// through the scalar unit as above, the next step's in flight. A
-// workgroup of sixteen waves runs on each CU (the host pads its LDS so that
-// no second one fits) and takes units cu, cu + G, cu + 2G, ... of the
-// launch's G workgroups, so that every CU has the same number of units to
-// within one, at most one more than the others on each SIMD.
+// The chunk's scores as units of one wave: (KV head, query head, 16 tokens,
+// 64 positions), the same dot chains as above. The products come from the
+// matrix unit: one v_mfma_f32_16x16x1_4b over zeros forms the 16 x 64
+// products of one dimension, each rounded as the reference's multiply (fma
+// with +0; a product of -0 becomes +0, which changes no sum, since no chain
+// ever is -0), and sixteen VALU adds put them on the chains. MFMA and VALU
+// share the SIMD's issue, but a product costs about 1/16 of an instruction
+// instead of one: 1.85 ns per 64 products and sums with two waves per SIMD,
+// against 2.6 at four for a multiply by a scalar and an add, and neither
+// operand passes through the scalar unit. Lane r holds the key of position
+// s0 + r (one slice of eight dimensions, two 16-byte loads, per eight
+// instructions) and the query of token r % 16; register 4 j + i of lane r is
+// position s0 + 16 j + 4 (r / 16) + i for token r % 16, so the scores are
+// stored 16 bytes at a time. A workgroup of sixteen waves runs on each CU (the
+// host pads its LDS so that no second one fits) and takes units cu, cu + G,
+// cu + 2G, ... of the launch's G workgroups, so that every CU has the same
+// number of units to within one, at most one more than the others on each
+// SIMD. Bound by that issue (107 cycles of a SIMD per dimension of a unit,
+// of 32 for the products and 64 for the sums at four cycles each): 512 tokens
+// of 2B over prefixes of 0, 512, 1024 and 1536 positions 23.4, 51.5, 79.8 and
+// 109 us a layer, 85 us on average before.
 constexpr int CSW_THREADS = 1024;
-constexpr uint32_t CSW_TOK = 8;
+constexpr uint32_t CSW_TOK = 16;
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ void chk_scores_unit(const dec_attn &A, uint32_t n_tok, uint32_t kvh, uint32_t hh,
                                                 uint32_t tb, uint32_t s0, uint32_t lane) {
-    const uint32_t grp = A.n_head / A.n_kv, hd = A.hd;
+    const uint32_t grp = A.n_head / A.n_kv, hd = A.hd, n_sl = hd / PV_SLICE;
     const uint32_t last_tok = min(tb + CSW_TOK, n_tok) - 1;
     const uint32_t npast_max = A.chunk_base + last_tok + 1;
-    // the lane's key (rows past the last token's position re-read a valid
-    // row): eight dimensions at krow, the next eight n_ctx * 8 floats on
+    // the lane's key and query (rows past the last ones re-read those): eight
+    // dimensions of the key at krow, the next eight n_ctx * 8 floats on
     const GLOBAL float *krow = G_CAST(const float, A.k_cache + ((size_t) kvh * A.n_ctx * hd +
                                                                 (size_t) min(s0 + lane, npast_max - 1) * PV_SLICE));
     const size_t kslice = (size_t) A.n_ctx * PV_SLICE;
-    typedef __attribute__((address_space(4))) const float cfloat;
-    typedef __attribute__((address_space(4))) const f32x4 cf32x4;
-    cfloat *qrow[CSW_TOK];
+    const GLOBAL float *qrow = G_CAST(const float, A.q + ((size_t) min(tb + lane % CSW_TOK, last_tok) * A.n_head +
+                                                          kvh * grp + hh) * hd);
+    auto load = [&](uint32_t sl, f32x4 (&k)[2], f32x4 (&q)[2]) {
+        const uint32_t c = min(sl, n_sl - 1);
 #pragma unroll
-    for (int tk = 0; tk < (int) CSW_TOK; ++tk)
-        qrow[tk] = (cfloat *) (A.q + ((size_t) min(tb + (uint32_t) tk, last_tok) * A.n_head + kvh * grp + hh) * hd);
-    float acc[CSW_TOK];
-#pragma unroll
-    for (int tk = 0; tk < (int) CSW_TOK; ++tk) acc[tk] = 0.0f;
-    auto qload = [&](uint32_t d0, f32x4 (&q)[CSW_TOK]) {
-#pragma unroll
-        for (int tk = 0; tk < (int) CSW_TOK; ++tk) q[tk] = *(cf32x4 *) (qrow[tk] + min(d0, hd - 4));
-    };
-    // four dimensions: the first product waits for this step's queries, then
-    // the next step's go out
-    auto step4 = [&](uint32_t d0, const f32x4 &k4, const f32x4 (&qc)[CSW_TOK], f32x4 (&qn)[CSW_TOK]) {
-        float a0 = acc[0] + qc[0][0] * k4[0];
-        __builtin_amdgcn_sched_barrier(0);
-        qload(d0 + 4, qn);
-        __builtin_amdgcn_sched_barrier(0);
-        a0 = a0 + qc[0][1] * k4[1];
-        a0 = a0 + qc[0][2] * k4[2];
-        acc[0] = a0 + qc[0][3] * k4[3];
-#pragma unroll
-        for (int tk = 1; tk < (int) CSW_TOK; ++tk) {
-            float a = acc[tk];
-            a = a + qc[tk][0] * k4[0];
-            a = a + qc[tk][1] * k4[1];
-            a = a + qc[tk][2] * k4[2];
-            acc[tk] = a + qc[tk][3] * k4[3];
+        for (int i = 0; i < 2; ++i) {
+            k[i] = *reinterpret_cast<const GLOBAL f32x4 *>(krow + c * kslice + 4 * i);
+            q[i] = *reinterpret_cast<const GLOBAL f32x4 *>(qrow + c * PV_SLICE + 4 * i);
         }
     };
-    const uint32_t n_ch = hd / 32u;                    // hd % 32 == 0
-    auto kload = [&](uint32_t ch, f32x4 (&k)[8]) {
-        const uint32_t sl = min(ch, n_ch - 1u) * 4u;     // four slices of eight dimensions
+    f32x16 acc = (f32x16) (0.0f);
+    auto slice = [&](const f32x4 (&k)[2], const f32x4 (&q)[2]) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-            k[i] = *reinterpret_cast<const GLOBAL f32x4 *>(krow + (sl + (uint32_t) i / 2u) * kslice + 4u * ((uint32_t) i & 1u));
-    };
-    // 32 dimensions; queries of its first step in qa on entry, of the next chunk's first step on exit
-    f32x4 qa[CSW_TOK], qb[CSW_TOK];
-    auto chunk = [&](uint32_t ch, const f32x4 (&k)[8]) {
+        for (int d = 0; d < 8; ++d) {
+            const f32x16 x = __builtin_amdgcn_mfma_f32_16x16x1f32(k[d / 4][d % 4], q[d / 4][d % 4], (f32x16) (0.0f), 0, 0, 0);
 #pragma unroll
-        for (int i = 0; i < 8; i += 2) {
-            step4(32u * ch + 4u * (uint32_t) i, k[i], qa, qb);
-            step4(32u * ch + 4u * (uint32_t) i + 4u, k[i + 1], qb, qa);
+            for (int r = 0; r < 16; ++r) acc[r] = acc[r] + x[r];
         }
     };
-    f32x4 ka[8], kb[8];
-    kload(0, ka);
-    qload(0, qa);
-    kload(1, kb);
-    uint32_t ch = 0;
-    for (; ch + 2 <= n_ch; ch += 2) {
-        chunk(ch, ka);
-        kload(ch + 2, ka);
-        chunk(ch + 1, kb);
-        kload(ch + 3, kb);
+    f32x4 ka[2], qa[2], kb[2], qb[2];
+    load(0, ka, qa);
+    load(1, kb, qb);
+    for (uint32_t sl = 0; sl < n_sl; sl += 2) {
+        slice(ka, qa);
+        load(sl + 2, ka, qa);
+        asm volatile("" ::: "memory");               // (not moved down to their use)
+        if (sl + 1 < n_sl) slice(kb, qb);            // uniform
+        load(sl + 3, kb, qb);
+        asm volatile("" ::: "memory");
     }
-    if (ch < n_ch) chunk(ch, ka);                      // an odd chunk count
-    if (s0 + lane < npast_max) {
 #pragma unroll
-        for (int tk = 0; tk < (int) CSW_TOK; ++tk) {
-            const uint32_t t = tb + (uint32_t) tk;
-            if (t < n_tok && s0 + lane <= A.chunk_base + t) {
-                A.scores[(size_t) t * A.n_head * A.sc_stride + (size_t) (kvh * grp + hh) * A.sc_stride + s0 + lane] =
-                    acc[tk] * A.attn_scale;
-            }
-        }
+    for (int r = 0; r < 16; ++r) acc[r] = acc[r] * A.attn_scale;
+    // a store's positions past the token's own (at most three, inside its row
+    // of sc_stride scores) are never read
+    const uint32_t t = tb + lane % CSW_TOK, s = s0 + 4 * (lane / CSW_TOK);
+    if (t >= n_tok) return;
+    GLOBAL float *row = G_CAST(float, A.scores) + ((size_t) t * A.n_head + kvh * grp + hh) * A.sc_stride;
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+        if (s + 16 * j <= A.chunk_base + t)
+            *reinterpret_cast<GLOBAL f32x4 *>(row + s + 16 * j) =
+                (f32x4) { acc[4 * j], acc[4 * j + 1], acc[4 * j + 2], acc[4 * j + 3] };
     }
 }
 
@@ -793,7 +774,7 @@ sllm_k_chk_scores_w(dec_attn A, uint32_t n_tok) {
     const uint32_t G = gridDim.x, cu = blockIdx.x, nkh = A.n_head;
     const uint32_t grp = A.n_head / A.n_kv;
     // lane j: token block j's position blocks (a chunk has at most 512
-    // tokens: 64 blocks), then their inclusive prefix sum over the lanes
+    // tokens: 32 blocks), then their inclusive prefix sum over the lanes
     const uint32_t n_tb = (n_tok + CSW_TOK - 1) / CSW_TOK;
     uint32_t inc = lane < n_tb ? (A.chunk_base + min(CSW_TOK * (lane + 1u), n_tok) + ATT_POS - 1) / ATT_POS : 0u;
 #pragma unroll
@@ -1657,7 +1638,6 @@ sllm_k_chk_kv_store(dec_attn A) {
 // the first.
 extern "C" __global__ void __launch_bounds__(CLM_THREADS, 2)
 sllm_k_chk_lm_head(chk_lm L) {
-    typedef float f32x16 __attribute__((ext_vector_type(16)));
     __shared__ __attribute__((aligned(1024))) uint8_t S[CLM_THREADS / 64 * CLM_RING * CLM_SLOT];
     const uint32_t n_tb = (L.n_tok + CLM_TOK - 1) / CLM_TOK;
     const uint32_t b = xcd_slot(L.n_wg);
@@ -2028,129 +2008,99 @@ sllm_k_chk_softmax(dec_attn A, uint32_t n_tok) {
     csm_full_row(A, row_i, lane, tab);
 }
 
-// The chunk's p . V in units of one wave: (KV head, query head h, half of
-// the head dimensions, 4 tokens), one dimension per lane. Each lane adds
-// p_s * v_s to four chains -- its dimension for the four tokens -- in order
-// of s (src/forward.c:706-726), a token's chain left alone past its own
-// position. p (written over the scores rows by sllm_k_chk_softmax) is the
-// same for every lane of a wave and comes through the scalar unit, eight
-// positions of a token per load; V rows stream from L2 two blocks of
-// sixteen positions ahead.
-constexpr uint32_t CP_TOK = 4;
+// The chunk's p . V in units of one wave: (KV head, query head h, 16 head
+// dimensions, 16 tokens). Each output is a chain, p_s * v_s added in order of
+// s (src/forward.c:706-726), left alone past its token's own position. The
+// products come from the matrix unit, as the scores': v_mfma_f32_16x16x1_4b
+// over zeros forms 16 dimensions x 16 tokens for four positions at a time.
+// Positions go in batches of sixteen: instruction i of four multiplies
+// positions 4 i .. 4 i + 3, lane 16 j + r giving V of dimension r at position
+// 4 i + j (each load is whole lines of two slices) and p of token r there (p,
+// written over the scores rows by sllm_k_chk_softmax, comes 16 bytes a lane,
+// positions 4 j .. 4 j + 3 of the batch, and is transposed over the four rows
+// of lanes), and register 4 j + k of the result is dimension 4 (lane / 16) + k
+// for token lane % 16, so each position is four adds. Units this small (5 a
+// SIMD for 512 tokens at 2B) can be dealt out evenly; with a whole 64
+// dimensions a unit, the longest one alone would take as long as the launch.
+// Loads past the caches' and rows' ends return zeros (buffer resources) and
+// those past a token's position are multiplied but never added. Bound as the scores are, and by
+// the latency of p, which only the Infinity Cache holds whole: with two, three
+// and four batches in flight 72.0, 64.9 and 69.2 us a layer on average over
+// the scores' four prefixes, 92 with products in the VALU and four tokens a
+// unit.
+constexpr uint32_t CP_TOK = 16, CP_DIM = 16, CP_BATCH = 16;
+constexpr int CP_RING = 3;              // batches in flight
 constexpr int CP_THREADS = 1024;
 
 __device__ __forceinline__ void chk_pv_unit(const dec_attn &A, uint32_t n_tok, uint32_t kvh, uint32_t tb,
-                                            uint32_t lane, uint32_t h, uint32_t half_id) {
-    const uint32_t grp = A.n_head / A.n_kv, hd = A.hd, ss = A.sc_stride;
-    const uint32_t last_tok = min(tb + CP_TOK, n_tok) - 1;
-    const uint32_t npast_max = A.chunk_base + last_tok + 1, npast_min = A.chunk_base + tb + 1;
-    const uint32_t d = min(64u * half_id + lane, hd - 1);
-    // dimension d of position s: slice d / 8, element d % 8
-    const float *vc = A.v_cache + ((size_t) kvh * (hd / PV_SLICE) + d / PV_SLICE) * A.n_ctx * PV_SLICE + d % PV_SLICE;
-    // p is not written during the launch: constant address space, so that
-    // its wave-uniform reads are scalar loads
-    typedef __attribute__((address_space(4))) const f32x8 cf32x8;
-    typedef __attribute__((address_space(4))) const float cfloat;
-    cfloat *prow[CP_TOK];                          // token rows past n_tok read the last one's
-    float acc[CP_TOK];
-    uint32_t npast_t[CP_TOK];                      // each token's own (past n_tok: never written out)
+                                            uint32_t lane, uint32_t h, uint32_t dq) {
+    const uint32_t grp = A.n_head / A.n_kv, hd = A.hd, ss = A.sc_stride, row = A.n_head * ss;
+    const uint32_t n_here = min(CP_TOK, n_tok - tb);
+    const uint32_t npast_min = A.chunk_base + tb + 1, npast_max = A.chunk_base + tb + n_here;
+    const uint32_t r = lane % 16, j4 = 4 * (lane / 16);
+    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
+        A.v_cache + (size_t) kvh * hd * A.n_ctx, (short) 0, (int) (hd * A.n_ctx * 4u), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
+        A.scores + (size_t) tb * row + (size_t) (kvh * grp + h) * ss, (short) 0,
+        (int) (((n_here - 1) * row + ss) * 4u), 0x00020000);
+    const uint32_t d = CP_DIM * dq + r;
+    uint32_t voff = ((d / PV_SLICE * A.n_ctx + lane / 16) * PV_SLICE + d % PV_SLICE) * 4u;
+    uint32_t poff = (min(r, n_here - 1) * row + j4) * 4u;
+    const uint32_t npast = r < n_here ? npast_min + r : 0u;
+    // the next batch's V and p
+    auto load = [&](float (&v)[4], u32x4 &p) {
 #pragma unroll
-    for (int tk = 0; tk < (int) CP_TOK; ++tk) {
-        prow[tk] = (cfloat *) (A.scores + ((size_t) min(tb + (uint32_t) tk, last_tok) * A.n_head + kvh * grp + h) * ss);
-        acc[tk] = 0.0f;
-        npast_t[tk] = A.chunk_base + tb + (uint32_t) tk + 1;
-    }
-    // p of positions s..s+7 of token tk (within the row: sc_stride >= n_ctx, a multiple of 8)
-    auto p8 = [&](int tk, uint32_t s) { return *(cf32x8 *) (prow[tk] + min(s, ss - 8)); };
-    float va[16], vb[16];
-    auto load16 = [&](uint32_t s, float (&v)[16]) {
-#pragma unroll
-        for (int q = 0; q < 16; ++q) v[q] = *G_CAST(const float, vc + (size_t) min(s + (uint32_t) q, npast_max - 1) * PV_SLICE);
+        for (int i = 0; i < 4; ++i)
+            v[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rv, (int) (voff + (uint32_t) i * 4u * PV_SLICE * 4u), 0, 0));
+        p = __builtin_amdgcn_raw_buffer_load_b128(rp, (int) poff, 0, 0);
+        voff += CP_BATCH * PV_SLICE * 4u;
+        poff += CP_BATCH * 4u;
     };
-    // eight positions at which every token of the block is live, with p of
-    // them in pc; the next eight's p go to pn. Scalar loads return out of
-    // order, so a wait covers all of them: the next loads are issued only
-    // after the first use of pc has waited for it.
-    auto step8 = [&](uint32_t s, const float *v, const f32x8 (&pc)[CP_TOK], f32x8 (&pn)[CP_TOK]) {
+    float acc[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
+    auto batch = [&](uint32_t s, const float (&v)[4], const u32x4 &p) {
+        // register i of lane row j (positions 4 j + i) to register j of row i
+        const auto a02 = __builtin_amdgcn_permlane32_swap(p[0], p[2], false, false);
+        const auto a13 = __builtin_amdgcn_permlane32_swap(p[1], p[3], false, false);
+        const auto b01 = __builtin_amdgcn_permlane16_swap(a02[0], a13[0], false, false);
+        const auto b23 = __builtin_amdgcn_permlane16_swap(a02[1], a13[1], false, false);
+        const float q[4] = { __uint_as_float(b01[0]), __uint_as_float(b01[1]), __uint_as_float(b23[0]),
+                             __uint_as_float(b23[1]) };
+        f32x16 x[4];
 #pragma unroll
-        for (int tk = 0; tk < (int) CP_TOK; ++tk) acc[tk] = acc[tk] + pc[tk][0] * v[0];
-        __builtin_amdgcn_sched_barrier(0);
+        for (int i = 0; i < 4; ++i) x[i] = __builtin_amdgcn_mfma_f32_16x16x1f32(v[i], q[i], (f32x16) (0.0f), 0, 0, 0);
+        if (s + CP_BATCH <= npast_min) {            // uniform: every token live
 #pragma unroll
-        for (int tk = 0; tk < (int) CP_TOK; ++tk) pn[tk] = p8(tk, s + 8);
-        __builtin_amdgcn_sched_barrier(0);
-        // per position the four products, then the four sums: no sum right
-        // behind the product it waits for (a wave alone on its SIMD)
+            for (int e = 0; e < 16; ++e) {
 #pragma unroll
-        for (int q = 1; q < 8; ++q) {
-            float x[CP_TOK];
+                for (int k = 0; k < 4; ++k) acc[k] = acc[k] + x[e / 4][e % 4 * 4 + k];
+            }
+        } else {
 #pragma unroll
-            for (int tk = 0; tk < (int) CP_TOK; ++tk) x[tk] = pc[tk][q] * v[q];
-            __builtin_amdgcn_sched_barrier(0);
+            for (int e = 0; e < 16; ++e) {
+                if (s + (uint32_t) e < npast) {
 #pragma unroll
-            for (int tk = 0; tk < (int) CP_TOK; ++tk) acc[tk] = acc[tk] + x[tk];
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-    f32x8 pa[CP_TOK], pb[CP_TOK];
-#pragma unroll
-    for (int tk = 0; tk < (int) CP_TOK; ++tk) pa[tk] = p8(tk, 0);
-    // sixteen positions: p of the first eight in pa on entry, of the next
-    // sixteen's first eight in pa on exit
-    auto step16 = [&](uint32_t s, const float (&v)[16]) {
-        step8(s, v, pa, pb);
-        step8(s + 8, v + 8, pb, pa);
-    };
-    // the last positions: a token's chain left alone past its own
-    auto tail = [&](uint32_t s, uint32_t r, const float (&v)[16]) {
-#pragma unroll
-        for (int hb = 0; hb < 2; ++hb) {
-            if (8u * (uint32_t) hb < r) {
-                f32x8 p[CP_TOK];
-#pragma unroll
-                for (int tk = 0; tk < (int) CP_TOK; ++tk) p[tk] = p8(tk, s + 8u * (uint32_t) hb);
-#pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    const uint32_t at = s + 8u * (uint32_t) hb + (uint32_t) q;
-                    if (8u * (uint32_t) hb + (uint32_t) q < r) {
-#pragma unroll
-                        for (int tk = 0; tk < (int) CP_TOK; ++tk) {
-                            const float x = p[tk][q] * v[8 * hb + q];
-                            acc[tk] = at < npast_t[tk] ? acc[tk] + x : acc[tk];
-                        }
-                    }
+                    for (int k = 0; k < 4; ++k) acc[k] = acc[k] + x[e / 4][e % 4 * 4 + k];
                 }
             }
         }
     };
-    load16(0, va);
-    load16(16, vb);
-    uint32_t s = 0;
-    const uint32_t end = npast_max;
-    const uint32_t bulk = min(end, npast_min);      // every token live before this
-    for (; s + 32 <= bulk; s += 32) {
-        step16(s, va);
-        load16(s + 32, va);
-        step16(s + 16, vb);
-        load16(s + 48, vb);
-    }
-    // at most 15 + 3 positions remain, in va then vb
-    if (s + 16 <= bulk) {
-        step16(s, va);
-        s += 16;
-        load16(s + 16, va);
-        tail(s, min(end - s, 16u), vb);
-        if (end - s > 16) tail(s + 16, end - s - 16, va);
-    } else {
-        tail(s, min(end - s, 16u), va);
-        if (end - s > 16) tail(s + 16, end - s - 16, vb);
-    }
-    if (64u * half_id + lane < hd) {
+    float v[CP_RING][4];
+    u32x4 p[CP_RING];
 #pragma unroll
-        for (int tk = 0; tk < (int) CP_TOK; ++tk) {
-            const uint32_t t = tb + (uint32_t) tk;
-            if (t < n_tok) A.out[(size_t) t * A.n_head * hd + (size_t) (kvh * grp + h) * hd + 64u * half_id + lane] = acc[tk];
+    for (int u = 0; u < CP_RING; ++u) load(v[u], p[u]);
+    for (uint32_t s = 0; s < npast_max; s += CP_RING * CP_BATCH) {
+#pragma unroll
+        for (int u = 0; u < CP_RING; ++u) {
+            const uint32_t at = s + (uint32_t) u * CP_BATCH;
+            if (at < npast_max) batch(at, v[u], p[u]);       // uniform
+            load(v[u], p[u]);
+            asm volatile("" ::: "memory");                   // (not moved down to their use)
         }
     }
+    const uint32_t t = tb + r, d0 = CP_DIM * dq + j4;
+    if (t < n_tok && d0 < hd)                        // hd % 8 == 0
+        *reinterpret_cast<GLOBAL f32x4 *>(G_CAST(float, A.out) + ((size_t) t * A.n_head + kvh * grp + h) * hd + d0) =
+            (f32x4) { acc[0], acc[1], acc[2], acc[3] };
 }
 
 // One workgroup of sixteen waves per CU (the host pads its LDS so that no
@@ -2170,8 +2120,8 @@ sllm_k_chk_pv(dec_attn A, uint32_t n_tok) {
     // HW_ID bits 5:4: the SIMD this wave runs on
     const uint32_t simd = __builtin_amdgcn_readfirstlane((__builtin_amdgcn_s_getreg(63492) >> 4) & 3u);
     const uint32_t n_simd = 4u * gridDim.x;
-    const uint32_t grp = A.n_head / A.n_kv, halves = (A.hd + 63u) / 64u;
-    const uint32_t per_tb = A.n_kv * grp * halves;                  // units per token block
+    const uint32_t grp = A.n_head / A.n_kv, dims = (A.hd + CP_DIM - 1) / CP_DIM;
+    const uint32_t per_tb = A.n_kv * grp * dims;                  // units per token block
     const uint32_t n_tb = (n_tok + CP_TOK - 1) / CP_TOK, n_units = per_tb * n_tb;
     for (uint32_t j = 0; j < 4u; ++j) {
         const uint32_t sm = (simd + j) & 3u, sig = 4u * blockIdx.x + sm;
@@ -2181,8 +2131,8 @@ sllm_k_chk_pv(dec_attn A, uint32_t n_tok) {
             r = __builtin_amdgcn_readfirstlane(r);
             const uint32_t k = r * n_simd + ((r & 1u) ? n_simd - 1u - sig : sig);
             if (k >= n_units) break;                                // uniform; later rounds are further out
-            const uint32_t rem = k % per_tb, kh = rem / halves;
-            chk_pv_unit(A, n_tok, kh / grp, (n_tb - 1u - k / per_tb) * CP_TOK, lane, kh % grp, rem % halves);
+            const uint32_t rem = k % per_tb, kh = rem / dims;
+            chk_pv_unit(A, n_tok, kh / grp, (n_tb - 1u - k / per_tb) * CP_TOK, lane, kh % grp, rem % dims);
         }
     }
 }
