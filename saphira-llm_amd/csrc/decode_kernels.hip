@@ -1727,12 +1727,17 @@ sllm_k_chk_lm_head(chk_lm L) {
 // of the groups (((e0+e4) + (e1+e5)) + (e2+e6)) + (e3+e7) and of the tail
 // terms in any order, checked, in the reference's order when the check
 // cannot decide; inv = 1/sum -- then p_s = e_s * inv written back over the
-// row for s < npast (e recomputed for rows past 512 positions: the same
+// row for s < npast (e recomputed for rows past 2048 positions: the same
 // bits).
 constexpr int CSM_THREADS = 256;        // four waves per workgroup
 
-// One row of at most 512 positions or more, a whole wave (lane l holds
-// positions 8l .. 8l + 7 of each block of 512)
+// One row, a whole wave (lane l holds positions 8l .. 8l + 7 of each block of
+// 512). NB blocks: the row's scores, then its exps, stay in registers, so the
+// row is read once, each exp formed once and p written once. NB = 0: a row of
+// any length, read and its exps formed again for the last pass (rows past
+// 2048 positions; taken for all rows past 512 positions, 512 tokens of 2B over a
+// prefix of 1536 took 53 us instead of 31).
+template <int NB>
 __device__ __forceinline__ void csm_full_row(const dec_attn &A, uint32_t row_i, uint32_t lane, const uint64_t *tab) {
     const uint32_t t = row_i / A.n_head, hh = row_i % A.n_head, ss = A.sc_stride;
     const uint32_t npast = A.chunk_base + t + 1, nb = npast / 8, nt = nb * 8;
@@ -1802,17 +1807,25 @@ __device__ __forceinline__ void csm_full_row(const dec_attn &A, uint32_t row_i, 
 
     float m = -INFINITY;
     double part = 0.0;
-    float v1[8];                                    // a row of one round stays in registers
-    if (npast <= 512) {
-        const uint32_t s = 8 * lane;
-        load8(s, v1);
+    float vr[NB > 0 ? NB : 1][8];
+    if constexpr (NB > 0) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) m = fmaxf(m, s + (uint32_t) i < npast ? v1[i] : -INFINITY);
+        for (int b = 0; b < NB; ++b) load8(512u * (uint32_t) b + 8 * lane, vr[b]);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const uint32_t s = 512u * (uint32_t) b + 8 * lane;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) m = fmaxf(m, s + (uint32_t) i < npast ? vr[b][i] : -INFINITY);
+        }
         m = wave_max(m);
-        if (has_tail) tail8(v1, nt / 8u, m);
-        if (s < npast) {
-            ggml8(v1, s, m);
-            add_group(part, v1, s);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const uint32_t b0 = 512u * (uint32_t) b, s = b0 + 8 * lane;
+            if (has_tail && nt >= b0 && nt - b0 < 512u) tail8(vr[b], (nt - b0) / 8u, m);   // uniform
+            if (s < npast) {
+                ggml8(vr[b], s, m);
+                add_group(part, vr[b], s);
+            }
         }
     } else {
         for (uint32_t b0 = 0; b0 < npast; b0 += 512) {
@@ -1854,9 +1867,12 @@ __device__ __forceinline__ void csm_full_row(const dec_attn &A, uint32_t row_i, 
         inv = lane_f(inv, 0);
     }
     // every lane's reads of the row are done (the wave reduced them above)
-    if (npast <= 512) {
-        const uint32_t s = 8 * lane;
-        if (s < npast) store8(s, v1, inv);
+    if constexpr (NB > 0) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const uint32_t s = 512u * (uint32_t) b + 8 * lane;
+            if (s < npast) store8(s, vr[b], inv);
+        }
     } else {
         for (uint32_t b0 = 0; b0 < npast; b0 += 512) {
             float v[8];
@@ -2005,7 +2021,11 @@ sllm_k_chk_softmax(dec_attn A, uint32_t n_tok) {
     }
     const uint32_t row_i = n_short + (w - w_short);
     if (row_i >= n_tok * A.n_head) return;          // uniform
-    csm_full_row(A, row_i, lane, tab);
+    const uint32_t npast = A.chunk_base + row_i / A.n_head + 1;      // uniform
+    if (npast <= 512) csm_full_row<1>(A, row_i, lane, tab);
+    else if (npast <= 1024) csm_full_row<2>(A, row_i, lane, tab);
+    else if (npast <= 2048) csm_full_row<4>(A, row_i, lane, tab);
+    else csm_full_row<0>(A, row_i, lane, tab);
 }
 
 // The chunk's p . V in units of one wave: (KV head, query head h, 16 head
