@@ -168,15 +168,28 @@ __device__ __forceinline__ int quant_one(float xs) {
 
 constexpr int QUANT_THREADS = 256;
 
-__device__ __forceinline__ void quant_row(const float *__restrict__ x, uint32_t n,
-                                          int8_t *__restrict__ q, act_t *__restrict__ act,
-                                          float *red_f, int *red_i) {
+// NV > 0: n % 4 == 0 and n <= 4 NV QUANT_THREADS; the row is read once, all
+// its loads in flight together, and held in registers between the max and the
+// rounding. NV = 0: any n, read twice.
+template <int NV>
+__device__ __forceinline__ void quant_row_n(const float *__restrict__ x, uint32_t n,
+                                            int8_t *__restrict__ q, act_t *__restrict__ act,
+                                            float *red_f, int *red_i) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const bool vec = (n & 3u) == 0;
 
     // pass 1: amax = max |x|. fmaxf drops NaN exactly as `a > amax` does.
     float m = 0.0f;
-    if (vec) {
+    f32x4 held[NV > 0 ? NV : 1];
+    if constexpr (NV > 0) {
+#pragma unroll
+        for (int u = 0; u < NV; ++u) held[u] = *G_CAST(const f32x4, x + min(4u * (uint32_t) (tid + u * QUANT_THREADS), n - 4));
+#pragma unroll
+        for (int u = 0; u < NV; ++u) {               // (a thread past the row holds its last values again)
+            const f32x4 v = held[u];
+            m = fmaxf(m, fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
+        }
+    } else if (vec) {
         for (uint32_t i = 4u * tid; i < n; i += 4u * QUANT_THREADS) {
             const f32x4 v = *G_CAST(const f32x4, x + i);
             m = fmaxf(m, fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
@@ -196,16 +209,22 @@ __device__ __forceinline__ void quant_row(const float *__restrict__ x, uint32_t 
 
     // pass 2: q = clamp(round-half-away(x*s)), running sum
     int sum = 0;
-    if (vec) {
-        for (uint32_t i = 4u * tid; i < n; i += 4u * QUANT_THREADS) {
-            const f32x4 v = *G_CAST(const f32x4, x + i);
-            const int a = quant_one(v[0] * s), b = quant_one(v[1] * s);
-            const int c = quant_one(v[2] * s), d = quant_one(v[3] * s);
-            sum += a + b + c + d;
-            *G_CAST(uint32_t, q + i) =
-                (uint32_t) (a & 0xff) | ((uint32_t) (b & 0xff) << 8) |
-                ((uint32_t) (c & 0xff) << 16) | ((uint32_t) (d & 0xff) << 24);
+    auto put4 = [&](uint32_t i, const f32x4 v) {
+        const int a = quant_one(v[0] * s), b = quant_one(v[1] * s);
+        const int c = quant_one(v[2] * s), d = quant_one(v[3] * s);
+        sum += a + b + c + d;
+        *G_CAST(uint32_t, q + i) =
+            (uint32_t) (a & 0xff) | ((uint32_t) (b & 0xff) << 8) |
+            ((uint32_t) (c & 0xff) << 16) | ((uint32_t) (d & 0xff) << 24);
+    };
+    if constexpr (NV > 0) {
+#pragma unroll
+        for (int u = 0; u < NV; ++u) {
+            const uint32_t i = 4u * (uint32_t) (tid + u * QUANT_THREADS);
+            if (i < n) put4(i, held[u]);
         }
+    } else if (vec) {
+        for (uint32_t i = 4u * tid; i < n; i += 4u * QUANT_THREADS) put4(i, *G_CAST(const f32x4, x + i));
     } else {
         for (uint32_t i = tid; i < n; i += QUANT_THREADS) {
             const int a = quant_one(G_CAST(const float, x)[i] * s);
@@ -223,6 +242,18 @@ __device__ __forceinline__ void quant_row(const float *__restrict__ x, uint32_t 
         G_CAST(float, act)[0] = s;
         G_CAST(int32_t, act)[1] = t;
     }
+}
+
+// One row by one workgroup. A batch of rows is bound by memory (5 bytes a
+// value, 4 read): 4096 rows of 6912 take 22.5 us (6.3 TB/s), 35 us when every
+// row was read twice; with few rows by one row's latency, 0.4 us less now.
+__device__ __forceinline__ void quant_row(const float *__restrict__ x, uint32_t n,
+                                          int8_t *__restrict__ q, act_t *__restrict__ act,
+                                          float *red_f, int *red_i) {
+    if ((n & 3u) != 0 || n > 16u * 4u * QUANT_THREADS) quant_row_n<0>(x, n, q, act, red_f, red_i);
+    else if (n <= 3u * 4u * QUANT_THREADS) quant_row_n<3>(x, n, q, act, red_f, red_i);
+    else if (n <= 7u * 4u * QUANT_THREADS) quant_row_n<7>(x, n, q, act, red_f, red_i);
+    else quant_row_n<16>(x, n, q, act, red_f, red_i);
 }
 
 // ---------------------------------------------------------------------------
