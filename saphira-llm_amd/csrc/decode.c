@@ -1131,12 +1131,8 @@ int sllm_gfx950_forward_chunk(const sllm_gfx950_model *m, sllm_gfx950_ctx *c, co
     if (st != SLLM_GFX950_OK) return st;
     c->n_past = base + n;
     c->have_logits = 1;
-    if (logits != NULL) {
-        he = hipMemcpyAsync(logits, c->chk.logits, (size_t) n * (size_t) m->n_vocab * 4, hipMemcpyDeviceToHost, s);
-        if (he == hipSuccess) he = hipStreamSynchronize(s);
-        if (he != hipSuccess) return sllm_shim_hip_fail(he, "forward_chunk: logits");
-    }
-    return SLLM_GFX950_OK;
+    return logits != NULL ? sllm_shim_d2h_pageable(logits, c->chk.logits, (size_t) n * (size_t) m->n_vocab * 4)
+                          : SLLM_GFX950_OK;
 }
 
 int sllm_gfx950_forward_prefill_chunked(const sllm_gfx950_model *m, sllm_gfx950_ctx *c, const int32_t *tokens,
