@@ -1427,7 +1427,12 @@ int sllm_shim_gemm_glu(const uint8_t *w_gate, const uint8_t *w_up, size_t n_rows
     k_gemm_args a;
     int tile = 0;
     uint64_t gx, gy;
-    const int st = gemm_prepare(jobs, 2, n, q, act, m, &a, &tile, &gx, &gy);
+    int st = gemm_prepare(jobs, 2, n, q, act, m, &a, &tile, &gx, &gy);
+    /* as for the QKV store: up to 64 tokens the 32 x 128 tile, for its
+     * silu(gate) * up: 1 to 6 us less a layer (67.7 -> 62.6 at 64 tokens). */
+    if (st == SLLM_GFX950_OK && gx != 0 && g.force_gemm_tile == 0 && tile != 9 && n % 256 == 0) {
+        st = gemm_prepare_tile(jobs, 2, n, q, act, m, 12, &a, &tile, &gx, &gy);
+    }
     if (st != SLLM_GFX950_OK || gx == 0) return st;
     const int which = n % 256 != 0 ? -1 : (tile == 12 ? 0 : (tile == 9 ? 1 : -1));
     if (which < 0) return SLLM_SHIM_NOT_FUSED;
