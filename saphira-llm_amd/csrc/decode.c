@@ -131,6 +131,7 @@ enum { IN_PLAIN = 0, IN_RESID = 1, IN_EMBED = 2, IN_SILU = 3 };
 #define CLM_ROWS     64
 #define CS_TOK       4    /* tokens per chunk scores workgroup, up to CS_SMALL tokens */
 #define CS_SMALL     128
+#define CSW_TOK      16   /* tokens per one-wave scores unit */
 #define CSW_THREADS  1024 /* the one-wave-unit scores kernel: sixteen waves per CU */
 #define CSW_LDS_PAD  98304u   /* its (unused) LDS: more than half a CU's, one workgroup per CU */
 #define CP_THREADS   1024 /* threads per chunk p.V workgroup: sixteen waves, one workgroup per CU */
@@ -992,8 +993,14 @@ static int launch_chunk(sllm_gfx950_ctx *c, int32_t n, int32_t base, int all_log
         if (st == SLLM_GFX950_OK) {
             uint32_t n_tok = (uint32_t) n;
             void *sargs[] = { &A, &n_tok };
-            if (n > CS_SMALL) {
-                /* units of one wave dealt evenly over one workgroup per CU */
+            /* units of one wave dealt evenly over one workgroup per CU: for
+             * every larger chunk, and for a small one over a prefix long
+             * enough for four units a CU (measured at 2B, a layer: 96 tokens
+             * over 512 positions 93.1 -> 88.4 us, 128 tokens 99.5 -> 93.6; 64
+             * tokens there no different, small chunks from position 0 four us
+             * slower) */
+            const uint64_t units = (uint64_t) ((n + CSW_TOK - 1) / CSW_TOK) * pos_blocks * (uint64_t) m->n_head;
+            if (n > CS_SMALL || units >= 4u * (uint64_t) cu_count()) {
                 st = sllm_shim_launch(c->f_cscores_w, cu_count(), 1, CSW_THREADS, CSW_LDS_PAD, sargs);
             } else {
                 /* four tokens per workgroup: the grid of a small chunk's units is too small */

@@ -40,7 +40,7 @@ def test_head_widths(amd, orc, dev, n_embd, n_head, n_head_kv, n_rot, n):
 
 
 @pytest.mark.parametrize("base,n,n_ctx", [(380, 140, 520), (505, 130, 640), (1000, 133, 1135), (1990, 129, 2119),
-                                          (2048, 145, 2200)])
+                                          (2048, 145, 2200), (3000, 99, 3100), (4000, 120, 4125)])
 def test_row_lengths(amd, orc, dev, base, n, n_ctx):
     print("[case] rows", base, n, flush=True)
     model = _model(amd, 128, 2, 1, 64, 32)
