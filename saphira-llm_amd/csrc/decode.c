@@ -135,6 +135,9 @@ enum { IN_PLAIN = 0, IN_RESID = 1, IN_EMBED = 2, IN_SILU = 3 };
 #define CSW_THREADS  1024 /* the one-wave-unit scores kernel: sixteen waves per CU */
 #define CSW_LDS_PAD  98304u   /* its (unused) LDS: more than half a CU's, one workgroup per CU */
 #define CP_THREADS   1024 /* threads per chunk p.V workgroup: sixteen waves, one workgroup per CU */
+#define CLR_THREADS  256
+#define CLR_BLOCK    1024   /* float4 per clearing workgroup */
+#define CLR_MAX_ROWS 32768u /* rows per clearing launch */
 #define CSM_WAVES    4    /* waves per chunk softmax workgroup */
 #define CSM_HALF     256  /* rows of at most this many positions take half a wave */
 /* sllm_k_chk_kv_store stages a token's query row (n_head * hd = n_embd floats) in 7168 floats of LDS */
@@ -322,7 +325,7 @@ struct sllm_gfx950_ctx {
     k_dec_lm      lm_args;
     size_t        kv_per_layer;    /* floats */
     hipFunction_t f_gemv, f_scores, f_pv, f_lm, f_argmax;
-    hipFunction_t f_prep, f_kvs, f_cscores4, f_cscores_w, f_csoft, f_cpv, f_clm, f_keys;
+    hipFunction_t f_prep, f_kvs, f_cscores4, f_cscores_w, f_csoft, f_cpv, f_clm, f_keys, f_clear;
     uint32_t      sc_stride;
     chunk_bufs    chk;
     int           graph_on, graph_ready;
@@ -536,7 +539,8 @@ int sllm_gfx950_ctx_new(const sllm_gfx950_model *m, int32_t n_ctx, sllm_gfx950_c
             (st = sllm_shim_decode_function("sllm_k_chk_softmax", &c->f_csoft)) == SLLM_GFX950_OK &&
             (st = sllm_shim_decode_function("sllm_k_chk_pv", &c->f_cpv)) == SLLM_GFX950_OK &&
             (st = sllm_shim_decode_function("sllm_k_chk_lm_head", &c->f_clm)) == SLLM_GFX950_OK &&
-            (st = sllm_shim_decode_function("sllm_k_chk_keys", &c->f_keys)) == SLLM_GFX950_OK) {
+            (st = sllm_shim_decode_function("sllm_k_chk_keys", &c->f_keys)) == SLLM_GFX950_OK &&
+            (st = sllm_shim_decode_function("sllm_k_dec_clear", &c->f_clear)) == SLLM_GFX950_OK) {
             st = sllm_shim_decode_function("sllm_k_dec_argmax", &c->f_argmax);
         }
     }
@@ -568,23 +572,31 @@ int32_t sllm_gfx950_ctx_n_past(const sllm_gfx950_ctx *c) { return c ? c->n_past 
 
 const float *sllm_gfx950_ctx_logits(const sllm_gfx950_ctx *c) { return c ? c->logits : NULL; }
 
+/* Zero positions [from, to) of every 8-dimension key and value slice. */
+static int clear_positions(sllm_gfx950_ctx *c, int32_t from, int32_t to) {
+    if (from >= to) return SLLM_GFX950_OK;
+    const uint32_t per_pos = PV_SLICE / 4;               /* float4 of a slice's position */
+    const uint32_t rows = (uint32_t) c->m->n_layer * (uint32_t) c->m->n_head_kv * (uint32_t) (c->m->hd / PV_SLICE);
+    float *k = c->k_cache, *v = c->v_cache;
+    uint32_t pitch = (uint32_t) c->n_ctx * per_pos, at = (uint32_t) from * per_pos, n = (uint32_t) (to - from) * per_pos;
+    int st = SLLM_GFX950_OK;
+    for (uint32_t r = 0; r < rows && st == SLLM_GFX950_OK; r += CLR_MAX_ROWS) {
+        float *kr = k + (size_t) r * pitch * 4, *vr = v + (size_t) r * pitch * 4;
+        void *args[] = { (void *) &kr, (void *) &vr, &pitch, &at, &n };
+        st = sllm_shim_launch_3d(c->f_clear, (n + CLR_BLOCK - 1) / CLR_BLOCK, rows - r < CLR_MAX_ROWS ? rows - r : CLR_MAX_ROWS,
+                                 2, CLR_THREADS, 0, args);
+    }
+    return st;
+}
+
 int sllm_gfx950_ctx_reset(sllm_gfx950_ctx *c) {
     DEC_NEED_OPEN();
     if (c == NULL) return sllm_shim_fail(SLLM_GFX950_ERR_ARG, "ctx_reset: NULL");
     const hipStream_t s = sllm_shim_stream();
-    hipError_t he = hipSuccess;
-    if (c->n_past > 0) {
-        /* the live prefix of every (layer, KV head): n_past positions of
-         * every 8-dimension key and value slice */
-        const size_t hd = (size_t) c->m->hd, rows = (size_t) c->m->n_layer * (size_t) c->m->n_head_kv;
-        he = hipMemset2DAsync(c->k_cache, (size_t) c->n_ctx * PV_SLICE * 4, 0, (size_t) c->n_past * PV_SLICE * 4,
-                              rows * (hd / PV_SLICE), s);
-        if (he == hipSuccess) {
-            he = hipMemset2DAsync(c->v_cache, (size_t) c->n_ctx * PV_SLICE * 4, 0, (size_t) c->n_past * PV_SLICE * 4,
-                                  rows * (hd / PV_SLICE), s);
-        }
-    }
-    if (he == hipSuccess) he = hipMemsetAsync(c->step, 0, sizeof(k_dec_step), s);
+    /* the live prefix of every (layer, KV head) */
+    const int st = clear_positions(c, 0, c->n_past);
+    if (st != SLLM_GFX950_OK) return st;
+    hipError_t he = hipMemsetAsync(c->step, 0, sizeof(k_dec_step), s);
     if (he == hipSuccess) he = hipStreamSynchronize(s);
     if (he != hipSuccess) return sllm_shim_hip_fail(he, "ctx_reset");
     c->n_past = 0;
@@ -839,12 +851,8 @@ int sllm_gfx950_ctx_kv_load(sllm_gfx950_ctx *c, const float *k, const float *v, 
     }
     /* positions past the restored prefix read as absent (zero) in every
      * (layer, KV head), as src/forward.c:1098-1118 clears them */
-    if (he == hipSuccess && n_pos < c->n_ctx) {
-        const size_t from = np * PV_SLICE * 4;
-        he = hipMemset2DAsync((uint8_t *) c->k_cache + from, pitch, 0, pitch - from, rows * n_sl, s);
-        if (he == hipSuccess) he = hipMemset2DAsync((uint8_t *) c->v_cache + from, pitch, 0, pitch - from, rows * n_sl, s);
-    }
-    if (he == hipSuccess && logits != NULL) {
+    int st = he == hipSuccess ? clear_positions(c, n_pos, c->n_ctx) : SLLM_GFX950_OK;
+    if (he == hipSuccess && st == SLLM_GFX950_OK && logits != NULL) {
         he = hipMemcpyAsync(c->logits, logits, (size_t) m->n_vocab * 4, hipMemcpyHostToDevice, s);
     }
     if (he != hipSuccess) {
@@ -852,8 +860,7 @@ int sllm_gfx950_ctx_kv_load(sllm_gfx950_ctx *c, const float *k, const float *v, 
         free(ks);
         return sllm_shim_hip_fail(he, "ctx_kv_load");
     }
-    int st = SLLM_GFX950_OK;
-    if (logits != NULL) {
+    if (st == SLLM_GFX950_OK && logits != NULL) {
         /* the restored logits' argmax becomes the step record's next token,
          * what an empty-prompt generate continues from (src/forward.c:909-912) */
         k_dec_step hs;

@@ -2191,3 +2191,21 @@ sllm_k_diag_expf(uint32_t first, uint32_t stride, uint32_t n, float *__restrict_
         out[i] = sllm_libm_expf(__uint_as_float(first + i * stride), tab);
     }
 }
+
+// Clear positions of both caches: `n` float4 from float4 `from` of every row
+// (a slice of eight dimensions of one KV head of one layer, pitch float4
+// long). Grid (blocks along the row, rows, 2 caches). Bound by the writes: the
+// runtime's strided fills took 390 us for 2048 positions of 2B (315 MB), and a
+// reset and prefill of them takes 0.7 ms less with this (31.96 -> 31.25 ms).
+constexpr int CLR_THREADS = 256, CLR_UNROLL = 4;
+
+extern "C" __global__ void __launch_bounds__(CLR_THREADS)
+sllm_k_dec_clear(float *__restrict__ k_cache, float *__restrict__ v_cache, uint32_t pitch, uint32_t from, uint32_t n) {
+    GLOBAL f32x4 *row = G_CAST(f32x4, blockIdx.z == 0 ? k_cache : v_cache) + (size_t) blockIdx.y * pitch + from;
+    const uint32_t i0 = blockIdx.x * (CLR_THREADS * CLR_UNROLL) + threadIdx.x;
+#pragma unroll
+    for (uint32_t u = 0; u < CLR_UNROLL; ++u) {
+        const uint32_t i = i0 + u * CLR_THREADS;
+        if (i < n) row[i] = (f32x4) { 0.0f, 0.0f, 0.0f, 0.0f };
+    }
+}
