@@ -159,7 +159,9 @@ int sllm_gfx950_gemv_epilogue(const uint8_t *w, size_t n_rows, size_t n,
  * K <= 16384 this is one launch: the slab (K <= 7168) or wide kernel quantises
  * x in LDS itself (the quantiser's operations, so the same bits); larger K
  * (or the streaming path forced with sllm_gfx950_set_tuning) runs a quantiser
- * launch first. */
+ * launch first, and so does 7168 < K <= 16384 where out, q or act overlaps
+ * x: there x has been read before anything is written. For K <= 7168 they must
+ * not overlap it. */
 int sllm_gfx950_linear(const uint8_t *w, size_t n_rows, size_t n, const float *x,
                        int8_t *q, sllm_gfx950_act *act, float *out);
 
@@ -170,7 +172,15 @@ int sllm_gfx950_linear(const uint8_t *w, size_t n_rows, size_t n, const float *x
  *              jobs sharing one x (Q/K/V, gate/up).
  *   x == NULL: q / act are inputs (act only needed for out).
  * out and/or rows_out may be NULL, not both. Device pointers, 16-byte
- * aligned. */
+ * aligned.
+ * Between jobs of K <= 7168 (and within one) nothing a job writes -- out,
+ * rows_out, and q / act beside an x -- may overlap what one reads: x, or q /
+ * act without one. Where a job of 7168 < K <= 16384 is the writer or the
+ * reader of such an overlap, the call's jobs of those K run as those of larger
+ * K do: every x of theirs is quantised, and the q / act beside it written,
+ * before any job's out or rows_out, so these may overlap x, and a job without
+ * x may take the q / act that another of them writes. Never may out or
+ * rows_out overlap a q / act that the call reads. */
 typedef struct sllm_gfx950_gemv_job {
     const uint8_t   *w;         /* whole packed tensor (codes + tail)    */
     size_t           n_rows;    /* N                                     */
@@ -184,9 +194,9 @@ typedef struct sllm_gfx950_gemv_job {
 
 /* Run independent GEMVs (Q, K and V against one activation, gate and up,
  * or many layers' matrices) in one launch when every K <= 7168 (else also a
- * launch for 7168 < K <= 16384, and a quantiser and a streaming launch above). The job tables are built and uploaded
- * on each call, and the call waits for the stream before freeing them; a
- * plan uploads them once. */
+ * launch for 7168 < K <= 16384, and a quantiser and a streaming launch
+ * above). The job tables are built and uploaded on each call, and the call
+ * waits for the stream before freeing them; a plan uploads them once. */
 int sllm_gfx950_gemv_batch(const sllm_gfx950_gemv_job *jobs, size_t n_jobs);
 
 /* Device memory of sllm_gfx950_gemv_batch_noalloc: a static array on each

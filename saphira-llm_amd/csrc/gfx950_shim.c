@@ -109,6 +109,7 @@ struct sllm_gfx950_plan {
     uint32_t   slab_wg, wide_wg;   /* multiples of 8 (empty descriptors pad them) */
     uint32_t   st_wg, st_lds, st_threads;
     int        st_lpr_idx;
+    int        wide_ok;        /* wide_allowed of the jobs */
     uint64_t   slab_target, wide_target;   /* bytes of packed weights per slab */
 };
 
@@ -766,13 +767,51 @@ static int slab_path(size_t n_rows, size_t k) {
     return (uint64_t) n_rows * (k / 4) + 32 <= 0xFFFF0000u;
 }
 
-/* which kernel a job of this shape takes */
+/* does a job have the shape of the wide kernel */
+static int wide_shape(size_t n_rows, size_t k) {
+    return g.force_path != 1 && k > SLAB_MAX_K && k <= WIDE_MAX_K && (uint64_t) n_rows * (k / 4) + 32 <= 0xFFFF0000u;
+}
+
+static int ranges_meet(const void *a, size_t a_bytes, const void *b, size_t b_bytes) {
+    return a != NULL && b != NULL && a_bytes != 0 && b_bytes != 0 && (uintptr_t) a < (uintptr_t) b + b_bytes &&
+           (uintptr_t) b < (uintptr_t) a + a_bytes;
+}
+
+/* does job a read anything that job b writes: its outputs, or the row it publishes */
+static int reads_written(const sllm_gfx950_gemv_job *a, const sllm_gfx950_gemv_job *b) {
+    const struct { const void *p; size_t n; }
+        rd[2] = { { a->x != NULL ? (const void *) a->x : (const void *) a->q, a->x != NULL ? a->n * 4 : a->n },
+                  { a->x != NULL ? NULL : (const void *) a->act, sizeof *a->act } },
+        wr[4] = { { b->out, b->n_rows * 4 }, { b->rows_out, b->n_rows * 4 },
+                  { b->x != NULL ? b->q : NULL, b->n }, { b->x != NULL ? b->act : NULL, sizeof *b->act } };
+    for (int i = 0; i < 2; ++i)
+        for (int o = 0; o < 4; ++o)
+            if (ranges_meet(rd[i].p, rd[i].n, wr[o].p, wr[o].n)) return 1;
+    return 0;
+}
+
+/*
+ * May the jobs of the wide shape take the wide kernel? Its workgroups read
+ * the activations while others of the launch already write, and the slab
+ * launch runs ahead of it; behind the quantiser launch every x has been read,
+ * and every q / act is there, before any output is written. So jobs of which
+ * one reads what another (or itself) writes, one of the two of the wide
+ * shape, keep the quantiser launch and the streaming kernel.
+ */
+static int wide_allowed(const sllm_gfx950_gemv_job *jobs, size_t n_jobs) {
+    for (size_t i = 0; i < n_jobs; ++i) {
+        if (!wide_shape(jobs[i].n_rows, jobs[i].n)) continue;
+        for (size_t j = 0; j < n_jobs; ++j)
+            if (reads_written(&jobs[i], &jobs[j]) || reads_written(&jobs[j], &jobs[i])) return 0;
+    }
+    return 1;
+}
+
+/* which kernel a job of this shape takes (wide_ok: wide_allowed of its launch's jobs) */
 enum { PATH_STREAM = 0, PATH_SLAB = 1, PATH_WIDE = 2 };
-static int job_path(size_t n_rows, size_t k) {
+static int job_path(size_t n_rows, size_t k, int wide_ok) {
     if (slab_path(n_rows, k)) return PATH_SLAB;
-    if (g.force_path != 1 && k > SLAB_MAX_K && k <= WIDE_MAX_K &&
-        (uint64_t) n_rows * (k / 4) + 32 <= 0xFFFF0000u) return PATH_WIDE;
-    return PATH_STREAM;
+    return wide_ok && wide_shape(n_rows, k) ? PATH_WIDE : PATH_STREAM;
 }
 
 /* chunks per lane of the wide kernel: 64 lanes of 16-byte chunks per row */
@@ -869,8 +908,8 @@ static int job_to_kernel(const sllm_gfx950_gemv_job *j, size_t i, k_gemv_job *kj
 static size_t align256(size_t v) { return (v + 255u) & ~(size_t) 255u; }
 
 /* streaming jobs that quantise x into plan scratch (carry x, no q / act) */
-static int takes_scratch(const sllm_gfx950_gemv_job *j) {
-    return j->x != NULL && j->q == NULL && job_path(j->n_rows, j->n) == PATH_STREAM;
+static int takes_scratch(const sllm_gfx950_gemv_job *j, int wide_ok) {
+    return j->x != NULL && j->q == NULL && job_path(j->n_rows, j->n, wide_ok) == PATH_STREAM;
 }
 
 /* scratch bytes for one quantised row of width k: q, then act */
@@ -878,12 +917,12 @@ static size_t row_scratch(size_t k) { return align256(k) + 256; }
 
 /* Bytes of plan scratch: one quantised row per distinct (x, K) among the
  * jobs that take scratch. */
-static size_t plan_scratch_bytes(const sllm_gfx950_gemv_job *jobs, size_t n_jobs) {
+static size_t plan_scratch_bytes(const sllm_gfx950_gemv_job *jobs, size_t n_jobs, int wide_ok) {
     size_t bytes = 0;
     for (size_t i = 0; i < n_jobs; ++i) {
-        if (!takes_scratch(&jobs[i])) continue;
+        if (!takes_scratch(&jobs[i], wide_ok)) continue;
         size_t e = 0;
-        while (e < i && !(takes_scratch(&jobs[e]) && jobs[e].x == jobs[i].x && jobs[e].n == jobs[i].n)) ++e;
+        while (e < i && !(takes_scratch(&jobs[e], wide_ok) && jobs[e].x == jobs[i].x && jobs[e].n == jobs[i].n)) ++e;
         if (e == i) bytes += row_scratch(jobs[i].n);
     }
     return bytes;
@@ -920,7 +959,7 @@ static int plan_layout(const sllm_gfx950_gemv_job *jobs, size_t n_jobs, sllm_gfx
         k_gemv_job *j = &kj[i];
         int st = job_to_kernel(&jobs[i], i, j);
         if (st != SLLM_GFX950_OK) return st;
-        path[i] = (uint8_t) job_path(j->n_rows, j->k);
+        path[i] = (uint8_t) job_path(j->n_rows, j->k, p->wide_ok);
         if (path[i] == PATH_SLAB) {
             j->variant = (uint32_t) slab_variant_for(j->k);
         } else if (path[i] == PATH_WIDE) {
@@ -1072,7 +1111,8 @@ int sllm_gfx950_plan_create(const sllm_gfx950_gemv_job *jobs, size_t n_jobs,
         st = fail(SLLM_GFX950_ERR_NOMEM, "plan: host tables");
     }
     if (st == SLLM_GFX950_OK) {
-        const size_t scratch = plan_scratch_bytes(jobs, n_jobs);
+        p->wide_ok = wide_allowed(jobs, n_jobs);
+        const size_t scratch = plan_scratch_bytes(jobs, n_jobs, p->wide_ok);
         if (scratch) {
             hipError_t e = hipMalloc(&p->scratch_dev, scratch);
             if (e != hipSuccess) st = hip_fail(e, "plan: activation scratch");
@@ -1168,7 +1208,8 @@ int sllm_gfx950_gemv_batch_noalloc(const sllm_gfx950_gemv_job *jobs, size_t n_jo
                     SLLM_GFX950_NOALLOC_MAX_JOBS);
     }
     const size_t cap = SLLM_GFX950_NOALLOC_SCRATCH_BYTES;
-    const size_t rows = align256(plan_scratch_bytes(jobs, n_jobs));
+    const int wide_ok = wide_allowed(jobs, n_jobs);
+    const size_t rows = align256(plan_scratch_bytes(jobs, n_jobs, wide_ok));
     if (rows > cap) {
         return fail(SLLM_GFX950_ERR_TOO_LARGE, "gemv_batch_noalloc: %zu bytes of quantised rows, the array holds %zu",
                     rows, cap);
@@ -1177,6 +1218,7 @@ int sllm_gfx950_gemv_batch_noalloc(const sllm_gfx950_gemv_job *jobs, size_t n_jo
     sllm_gfx950_plan p;
     memset(&p, 0, sizeof p);
     p.scratch_dev = g.noalloc_dev;
+    p.wide_ok = wide_ok;
     int st = plan_layout(jobs, n_jobs, &p, g_noalloc.quant, g_noalloc.jobs, g_noalloc.path);
     if (st == SLLM_GFX950_OK) {
         const size_t qbytes = p.n_quant * sizeof(k_quant_job), jbytes = n_jobs * sizeof(k_gemv_job);
@@ -1214,7 +1256,7 @@ static int single_launch(const sllm_gfx950_gemv_job *j) {
     const k_gemv_job *no_jobs = NULL;
     const k_wg_desc *no_descs = NULL;
     uint32_t zero = 0;
-    const int path = job_path(kj.n_rows, kj.k);
+    const int path = job_path(kj.n_rows, kj.k, wide_allowed(j, 1));
     if (path != PATH_STREAM) {
         const int wide = path == PATH_WIDE;
         kj.variant = wide ? wide_variant(kj.k) : (uint32_t) slab_variant_for(kj.k);
@@ -1243,7 +1285,7 @@ static int single_launch(const sllm_gfx950_gemv_job *j) {
     }
     const stream_shape ss = stream_shape_for();
     uint32_t rows;
-    const uint32_t wg = job_workgroups(&kj, 0, &rows, slab_default_target());
+    const uint32_t wg = job_workgroups(&kj, PATH_STREAM, &rows, slab_default_target());
     void *args[] = { (void *) &no_jobs, (void *) &no_descs, &zero, &kj, &rows };
     return launch(g.k_stream[ss.lpr_idx], wg, (uint32_t) (64 * ss.waves), kj.k, args);
 }

@@ -19,6 +19,8 @@
  *   fakehip_live()               resources held: memory, modules, streams,
  *                                events, graphs
  *   fakehip_calls()              HIP calls made so far
+ *   fakehip_launches()           names of the kernels launched since the last
+ *                                fakehip_clear, a space behind each
  */
 #include <hip/hip_runtime_api.h>
 
@@ -35,6 +37,8 @@ static long     g_fail_skip = -1;     /* < 0: disarmed */
 static int      g_fired;
 static long     g_live;
 static unsigned long g_calls;
+static char     g_launches[4096];     /* (names past its end are dropped) */
+static size_t   g_launches_len;
 
 FAKE_EXPORT void fakehip_fail(const char *fn, int err, unsigned skip) {
     snprintf(g_fail_fn, sizeof g_fail_fn, "%s", fn);
@@ -42,7 +46,8 @@ FAKE_EXPORT void fakehip_fail(const char *fn, int err, unsigned skip) {
     g_fail_skip = (long) skip;
     g_fired = 0;
 }
-FAKE_EXPORT void fakehip_clear(void) { g_fail_skip = -1; g_fired = 0; }
+FAKE_EXPORT void fakehip_clear(void) { g_fail_skip = -1; g_fired = 0; g_launches[g_launches_len = 0] = 0; }
+FAKE_EXPORT const char *fakehip_launches(void) { return g_launches; }
 FAKE_EXPORT int  fakehip_fired(void) { return g_fired; }
 FAKE_EXPORT long fakehip_live(void) { return g_live; }
 FAKE_EXPORT unsigned long fakehip_calls(void) { return g_calls; }
@@ -159,6 +164,9 @@ hipError_t hipModuleLaunchKernel(hipFunction_t f, unsigned int gx, unsigned int 
     (void) gx; (void) gy; (void) gz; (void) bx; (void) by; (void) bz; (void) lds; (void) s; (void) extra;
     INJECT();
     const char *name = ((const fake_fn *) f)->name;
+    if (g_launches_len + strlen(name) + 2 <= sizeof g_launches) {
+        g_launches_len += (size_t) snprintf(g_launches + g_launches_len, sizeof g_launches - g_launches_len, "%s ", name);
+    }
     if (strcmp(name, "sllm_k_host_done") == 0) {
         **(uint32_t **) args[0] = *(uint32_t *) args[1];
     } else if (strcmp(name, "sllm_k_quant_host") == 0) {

@@ -60,7 +60,7 @@ def fake(amd):
     L = amd._bind(FAKE, amd.PROTOTYPES)
     for name, res, args in (("fakehip_fail", None, [c_char_p, c_int, c_uint]), ("fakehip_clear", None, []),
                             ("fakehip_fired", c_int, []), ("fakehip_live", c_long, []),
-                            ("fakehip_calls", c_ulong, [])):
+                            ("fakehip_calls", c_ulong, []), ("fakehip_launches", c_char_p, [])):
         f = getattr(L, name)
         f.restype, f.argtypes = res, args
     yield L

@@ -61,3 +61,24 @@ def test_plan_of_every_kernel(amd, orc, dev, slab_kib):
             np.testing.assert_array_equal(b[3].download(np.int8, n), q, err_msg=f"job {i}")
         for v in b:
             v.free()
+
+
+def test_outputs_over_inputs_are_ordered(amd, orc, dev):
+    """out over its own x, and a job that takes the row another one publishes:
+    what the quantiser launch and the streaming kernel make of them."""
+    n_rows, n = 4099, 8192
+    w = amd.synth_i2s(amd.synth_seed(13, 0, 0, 0), n_rows, n)
+    x = amd.synth_normal(77, n)
+    y_o, q_o, _, _, _ = orc.linear(w, n_rows, n, x, orc.DOT_V3)
+    bw, bx, bq, ba, b1, b2 = dev.put(w), dev.put(x), dev.alloc(n), dev.alloc(8), dev.alloc(4 * n_rows), dev.alloc(4 * n_rows)
+    try:
+        dev.gemv_batch([amd.GemvJob(bw.ptr, n_rows, n, None, bq.ptr, ba.ptr, b2.ptr, None),
+                        amd.GemvJob(bw.ptr, n_rows, n, bx.ptr, bq.ptr, ba.ptr, b1.ptr, None)])
+        dev.linear(bw.vp, n_rows, n, bx.vp, None, None, bx.vp)
+        dev.sync()
+        np.testing.assert_array_equal(bq.download(np.int8, n), q_o)
+        for b in (b1, b2, bx):
+            np.testing.assert_array_equal(b.download(np.uint32, n_rows), y_o.view(np.uint32))
+    finally:
+        for b in (bw, bx, bq, ba, b1, b2):
+            b.free()
