@@ -767,9 +767,11 @@ static int slab_path(size_t n_rows, size_t k) {
     return (uint64_t) n_rows * (k / 4) + 32 <= 0xFFFF0000u;
 }
 
-/* does a job have the shape of the wide kernel */
+/* does a job have the shape of the wide kernel (one without rows has no
+ * workgroup there to publish its q / act; the quantiser launch does) */
 static int wide_shape(size_t n_rows, size_t k) {
-    return g.force_path != 1 && k > SLAB_MAX_K && k <= WIDE_MAX_K && (uint64_t) n_rows * (k / 4) + 32 <= 0xFFFF0000u;
+    return g.force_path != 1 && n_rows > 0 && k > SLAB_MAX_K && k <= WIDE_MAX_K &&
+           (uint64_t) n_rows * (k / 4) + 32 <= 0xFFFF0000u;
 }
 
 static int ranges_meet(const void *a, size_t a_bytes, const void *b, size_t b_bytes) {

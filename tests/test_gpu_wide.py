@@ -82,3 +82,17 @@ def test_outputs_over_inputs_are_ordered(amd, orc, dev):
     finally:
         for b in (bw, bx, bq, ba, b1, b2):
             b.free()
+
+
+def test_job_without_rows_publishes_its_row(amd, orc, dev):
+    n = 8192
+    w = amd.synth_i2s(amd.synth_seed(14, 0, 0, 0), 16, n)
+    x = amd.synth_normal(78, n)
+    _, q_o, _, s_o, t_o = orc.linear(w, 16, n, x, orc.DOT_V3)
+    bufs = bw, bx, bq, ba, by = dev.put(w), dev.put(x), dev.put(np.full(n, 99, np.int8)), dev.alloc(8), dev.alloc(64)
+    dev.gemv_batch([amd.GemvJob(bw.ptr, 0, n, bx.ptr, bq.ptr, ba.ptr, by.ptr, None)])
+    np.testing.assert_array_equal(bq.download(np.int8, n), q_o)
+    a = ba.download(np.uint8, 8).view(np.dtype([("scale", "<f4"), ("sum", "<i4")]))[0]
+    assert a["scale"] == s_o and a["sum"] == t_o
+    for b in bufs:
+        b.free()

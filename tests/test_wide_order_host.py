@@ -108,3 +108,13 @@ def test_jobs_that_depend_on_each_other(amd, lib):
     # one job's out over another's x
     assert _batches(amd, lib, [amd.GemvJob(w, N, K, x, None, None, o1, None),
                                amd.GemvJob(w, N, K, o1, None, None, o2, None)]) == ordered + [STREAM]
+
+
+def test_job_without_rows_publishes_its_row(amd, lib):
+    """No rows, but q / act to write: the quantiser launch writes them (the
+    wide kernel would leave before it does)."""
+    m = Mem()
+    w, x, q, act, out = (m.at(v) for v in (400000, 0, 65536, 131072, 200000))
+    assert _batches(amd, lib, [amd.GemvJob(w, 0, K, x, q, act, out, None)]) == ["sllm_k_quant_list"]
+    assert _batches(amd, lib, [amd.GemvJob(w, 0, K, x, q, act, out, None),
+                               amd.GemvJob(w, N, K, x, None, None, out, None)]) == ["sllm_k_quant_list", WIDE]
