@@ -1145,7 +1145,7 @@ int sllm_gfx950_forward_chunk(const sllm_gfx950_model *m, sllm_gfx950_ctx *c, co
     if (st != SLLM_GFX950_OK) return st;
     c->n_past = base + n;
     c->have_logits = 1;
-    return logits != NULL ? sllm_shim_d2h_pageable(logits, c->chk.logits, (size_t) n * (size_t) m->n_vocab * 4)
+    return logits != NULL ? sllm_shim_d2h_host(logits, c->chk.logits, (size_t) n * (size_t) m->n_vocab * 4)
                           : SLLM_GFX950_OK;
 }
 

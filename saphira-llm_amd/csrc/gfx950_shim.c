@@ -543,7 +543,7 @@ int sllm_shim_launch_3d(hipFunction_t f, uint32_t gx, uint32_t gy, uint32_t gz, 
 }
 
 /* ------------------------------------------------------------------ */
-/* large results to pageable host memory                               */
+/* large results to host memory                                        */
 /* ------------------------------------------------------------------ */
 
 /*
@@ -559,7 +559,9 @@ int sllm_shim_launch_3d(hipFunction_t f, uint32_t gx, uint32_t gy, uint32_t gz, 
  *
  * The buffers are made by the first such copy, serve one copy at a time and
  * are freed by sllm_gfx950_close. Without them (no pinned memory to be had)
- * the plain copy runs.
+ * the plain copy runs, and to a destination that is pinned already: the pieces
+ * and their memcpy only delay it (128 tokens through 4 layers of 2B, the
+ * 65.7 MB of logits pinned: 2.93 -> 2.59 ms).
  */
 #define D2H_STAGED  (8u << 20)
 #define D2H_PIECE   (4u << 20)
@@ -629,10 +631,18 @@ static void d2h_free(void) {
     pthread_mutex_unlock(&g_d2h.mtx);
 }
 
-int sllm_shim_d2h_pageable(void *dst, const void *src, size_t bytes) {
+/* memory the runtime knows (pinned, managed): one copy reaches it at full rate */
+static int runtime_memory(const void *p) {
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, p) == hipSuccess) return at.type != hipMemoryTypeUnregistered;
+    (void) hipGetLastError();        /* not left for the caller's next HIP call */
+    return 0;
+}
+
+int sllm_shim_d2h_host(void *dst, const void *src, size_t bytes) {
     int staged = 0;
     hipError_t e = hipSuccess;
-    if (bytes >= D2H_STAGED) {
+    if (bytes >= D2H_STAGED && !runtime_memory(dst)) {
         pthread_mutex_lock(&g_d2h.mtx);
         staged = d2h_ready();
         if (staged) {

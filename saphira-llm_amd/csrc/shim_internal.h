@@ -53,9 +53,9 @@ _Static_assert(sizeof(k_wg_desc) == 16, "k_wg_desc must match wg_desc in i2s_dev
 SLLM_HIDDEN int      sllm_shim_slab_variant(uint32_t k);
 SLLM_HIDDEN uint32_t sllm_shim_slab_group_rows(int variant);
 
-/* Copy device memory, once the library stream reaches the copy, to pageable
- * host memory; returns with the bytes there (or a status). */
-SLLM_HIDDEN int         sllm_shim_d2h_pageable(void *dst, const void *src, size_t bytes);
+/* Copy device memory, once the library stream reaches the copy, to host
+ * memory, pageable or pinned; returns with the bytes there (or a status). */
+SLLM_HIDDEN int         sllm_shim_d2h_host(void *dst, const void *src, size_t bytes);
 SLLM_HIDDEN int         sllm_shim_is_open(void);
 SLLM_HIDDEN hipStream_t sllm_shim_stream(void);
 SLLM_HIDDEN int         sllm_shim_cu(void);

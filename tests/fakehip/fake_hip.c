@@ -92,14 +92,34 @@ hipError_t hipMalloc(void **p, size_t bytes) {
     return *p ? hipSuccess : hipErrorOutOfMemory;
 }
 hipError_t hipFree(void *p) { ++g_calls; return fake_release(p); }
+/* pinned memory, for hipPointerGetAttributes (past the table: not known) */
+static struct { const uint8_t *p; size_t bytes; } g_pinned[64];
 hipError_t hipHostMalloc(void **p, size_t bytes, unsigned int flags) {
     (void) flags;
     *p = NULL;
     INJECT();
     *p = fake_alloc(bytes);
+    for (size_t i = 0; *p != NULL && i < sizeof g_pinned / sizeof *g_pinned; ++i) {
+        if (g_pinned[i].p == NULL) { g_pinned[i].p = *p; g_pinned[i].bytes = bytes; break; }
+    }
     return *p ? hipSuccess : hipErrorOutOfMemory;
 }
-hipError_t hipHostFree(void *p) { ++g_calls; return fake_release(p); }
+hipError_t hipHostFree(void *p) {
+    ++g_calls;
+    for (size_t i = 0; i < sizeof g_pinned / sizeof *g_pinned; ++i) if (g_pinned[i].p == p) g_pinned[i].p = NULL;
+    return fake_release(p);
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p) {
+    INJECT();
+    memset(a, 0, sizeof *a);
+    a->type = hipMemoryTypeUnregistered;
+    for (size_t i = 0; i < sizeof g_pinned / sizeof *g_pinned; ++i) {
+        const uint8_t *b = g_pinned[i].p;
+        if (b != NULL && (const uint8_t *) p >= b && (const uint8_t *) p < b + g_pinned[i].bytes) a->type = hipMemoryTypeHost;
+    }
+    return hipSuccess;
+}
+hipError_t hipGetLastError(void) { ++g_calls; return hipSuccess; }
 hipError_t hipHostGetDevicePointer(void **d, void *h, unsigned int flags) {
     (void) flags;
     INJECT();

@@ -1,9 +1,10 @@
-"""Large results on their way to pageable host memory, on the CPU: the
-library's C sources against the host-memory HIP stand-in. The copy goes
+"""Large results on their way to host memory, on the CPU: the library's C
+sources against the host-memory HIP stand-in. To pageable memory the copy goes
 through pinned pieces and several threads; a failing call reaches the caller
 as a status and leaves the copy usable; without pinned memory the plain copy
-runs; closing the library gives everything back."""
-from ctypes import byref, c_void_p
+runs, and to memory that is pinned already; closing the library gives everything
+back."""
+from ctypes import POINTER, byref, c_float, c_size_t, c_void_p, cast
 
 import numpy as np
 
@@ -46,6 +47,24 @@ def test_staged_copy_statuses_and_release(amd, fake):  # noqa: F811
             L.fakehip_clear()
             assert chunk() == 0 and not logits.any()
             assert L.fakehip_live() == live
+    # pinned by the caller: one plain copy, no event and no piece
+    pin = c_void_p()
+    assert L.hipHostMalloc(byref(pin), c_size_t(4 * N * VOCAB), 0) == 0
+    for at in (0, 4096):
+        rows = N if at == 0 else N - 1
+        held = np.ctypeslib.as_array(cast(pin.value + at, POINTER(c_float)), (rows * VOCAB,))
+        held.fill(7.0)
+        assert L.sllm_gfx950_ctx_reset(c) == 0
+        L.fakehip_fail(b"hipEventRecord", HIP_INVALID_VALUE, 0)
+        assert L.sllm_gfx950_forward_chunk(m, c, P(tokens), rows, 0, pin.value + at) == 0, _err(L)
+        assert not L.fakehip_fired() and not held.any()
+        L.fakehip_clear()
+    del held
+    assert L.hipHostFree(pin) == 0
+    # a runtime that cannot say what the memory is: staged, as pageable
+    L.fakehip_fail(b"hipPointerGetAttributes", HIP_INVALID_VALUE, 0)
+    assert chunk() == 0 and L.fakehip_fired() and not logits.any()
+    L.fakehip_clear()
     L.sllm_gfx950_ctx_free(c)
     L.sllm_gfx950_model_free(m)
     L.sllm_gfx950_close()

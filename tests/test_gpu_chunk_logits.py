@@ -1,6 +1,9 @@
 """Chunks whose logits are large enough to reach the host in pinned pieces by
 several threads: every row against the oracle's, bit for bit, at sizes on and
-off the piece, into fresh memory each time, from two contexts in turn."""
+off the piece, into fresh memory each time, from two contexts in turn; and into
+memory that is pinned already, which takes one copy."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -27,3 +30,27 @@ def test_large_logits(amd, orc, dev, n_vocab, n):
         got[i] = g.forward_chunk(toks, 0)
         np.testing.assert_array_equal(got[i].view(np.uint32), want.view(np.uint32))
         g.close()
+
+
+def _hip():
+    """The HIP runtime that the library is linked to, as loaded."""
+    with open("/proc/self/maps") as f:
+        return ctypes.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
+
+
+def test_large_logits_into_pinned_memory(amd, orc, dev):
+    n_vocab, n = 32769, 65
+    model = amd.synth_model(dict(CFG, n_vocab=n_vocab), 6)
+    toks = np.random.default_rng(n).integers(0, n_vocab, n).astype(np.int32)
+    o, g = orc.Decoder(model, n), amd.DeviceDecoder(dev, model, n)
+    want = np.stack([o.forward(int(t), i) for i, t in enumerate(toks)])
+    o.close()
+    hip, pin, off = _hip(), ctypes.c_void_p(), 4100
+    assert hip.hipHostMalloc(ctypes.byref(pin), ctypes.c_size_t(want.nbytes + off), 0) == 0
+    try:
+        assert amd.lib().sllm_gfx950_forward_chunk(g.m, g.c, amd.ptr(toks), n, 0, ctypes.c_void_p(pin.value + off)) == 0
+        got = np.ctypeslib.as_array(ctypes.cast(pin.value + off, ctypes.POINTER(ctypes.c_uint32)), want.shape)
+        np.testing.assert_array_equal(got, want.view(np.uint32))
+    finally:
+        g.close()
+        assert hip.hipHostFree(pin) == 0
