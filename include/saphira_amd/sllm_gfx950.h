@@ -156,12 +156,12 @@ int sllm_gfx950_gemv_epilogue(const uint8_t *w, size_t n_rows, size_t n,
 /* One projection as src/forward.c:651-655 performs it: quantise x (n
  * floats), GEMV, epilogue into out (n_rows floats). q / act, when not NULL,
  * receive the quantised row and its scale/sum (give both or neither). For
- * K <= 16384 this is one launch: the slab (K <= 7168) or wide kernel quantises
- * x in LDS itself (the quantiser's operations, so the same bits); larger K
- * (or the streaming path forced with sllm_gfx950_set_tuning) runs a quantiser
- * launch first, and so does 7168 < K <= 16384 where out, q or act overlaps
- * x: there x has been read before anything is written. For K <= 7168 they must
- * not overlap it. */
+ * K <= 7168, and up to 16384 where the tensor has at most 544 KiB a CU (136
+ * MiB), this is one launch: the slab or wide kernel quantises x in LDS itself
+ * (the quantiser's operations, so the same bits); larger ones (or the streaming
+ * path forced with sllm_gfx950_set_tuning) run a quantiser launch first, and
+ * so does 7168 < K <= 16384 where out, q or act overlaps x: there x has been
+ * read before anything is written. For K <= 7168 they must not overlap it. */
 int sllm_gfx950_linear(const uint8_t *w, size_t n_rows, size_t n, const float *x,
                        int8_t *q, sllm_gfx950_act *act, float *out);
 
@@ -195,7 +195,8 @@ typedef struct sllm_gfx950_gemv_job {
 /* Run independent GEMVs (Q, K and V against one activation, gate and up,
  * or many layers' matrices) in one launch when every K <= 7168 (else also a
  * launch for 7168 < K <= 16384, and a quantiser and a streaming launch
- * above). The job tables are built and uploaded on each call, and the call
+ * above, which the jobs of those K take too where they are too many or too
+ * large to run side by side). The job tables are built and uploaded on each call, and the call
  * waits for the stream before freeing them; a plan uploads them once. */
 int sllm_gfx950_gemv_batch(const sllm_gfx950_gemv_job *jobs, size_t n_jobs);
 
@@ -307,7 +308,8 @@ int sllm_gfx950_set_gemm_tile(int tile);
 /* Launch-geometry override for tuning sweeps and tests; affects launches
  * and plans created afterwards. All zero (variant -1) is automatic.
  *   path           0 auto and 2: slab kernel for K <= 7168, wide kernel up to
- *                  16384, streaming kernel above; 1: streaming kernel for every K
+ *                  16384 where its workgroups all run at once, else the
+ *                  streaming kernel; 1: streaming kernel for every K
  *   variant        slab geometry: 0 (8 lanes x 5 chunks per row) or 1
  *                  (16 x 7), used when it covers K; -1 auto
  *   lanes_per_row  streaming kernel: 4, 8 or 16

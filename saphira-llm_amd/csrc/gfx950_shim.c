@@ -109,8 +109,8 @@ struct sllm_gfx950_plan {
     uint32_t   slab_wg, wide_wg;   /* multiples of 8 (empty descriptors pad them) */
     uint32_t   st_wg, st_lds, st_threads;
     int        st_lpr_idx;
-    int        wide_ok;        /* wide_allowed of the jobs */
-    uint64_t   slab_target, wide_target;   /* bytes of packed weights per slab */
+    uint64_t   slab_target;    /* bytes of packed weights per slab */
+    uint64_t   wide_target;    /* the same of the wide jobs; 0: they are streaming jobs */
 };
 
 static struct {
@@ -728,12 +728,13 @@ int sllm_gfx950_quant_act(const float *x, size_t n, size_t n_tok, int8_t *q,
  * (K <= 2560), variant 1 16 lanes x 7 chunks (K <= 7168). A job carrying
  * f32 x is quantised inside the kernel: no quantiser launch.
  *
- * Wide kernel (SLAB_MAX_K < K <= WIDE_MAX_K): the slab kernel's scheme with
+ * Wide kernel (SLAB_MAX_K < K <= WIDE_MAX_K, within the bounds of wide_fit and
+ * wide_ordered): the slab kernel's scheme with
  * sixteen waves, one row per wave and pass, so groups of 16 rows, up to the
  * K that four chunks a lane cover. One launch where the streaming kernel
  * takes two; 4096 x 14336 from f32 x: 8.0 us against 22.0.
  *
- * Streaming kernel (larger K, or forced with path 1): LPR lanes per row, W
+ * Streaming kernel (all others, or forced with path 1): LPR lanes per row, W
  * waves looping over groups of 64/LPR rows inside a slab of rows_per_wg rows,
  * reading a quantised row staged in LDS; jobs carrying f32 x are quantised
  * first, by one list-quantiser launch per batch.
@@ -748,7 +749,8 @@ int sllm_gfx950_quant_act(const float *x, size_t n, size_t n_tok, int8_t *q,
 #define WIDE_THREADS     1024
 #define WIDE_MAX_K       16384
 #define WIDE_GROUP       16u     /* rows per pass: one per wave */
-#define WIDE_KIB         544     /* largest slab of a batch: 136 KiB per four waves, as the slab kernel's */
+#define WIDE_KIB         544     /* weights a workgroup, at most: 136 KiB per four waves, as the slab kernel's */
+#define WIDE_SLACK_KIB   128     /* a batch's largest slab above its average, at most; twice that with an x to quantise */
 #define SLAB_DEFAULT_KIB 136     /* 32 slabs per BitNet-2B FFN matrix: 2-4 % faster than 34 (128 KiB) */
 
 typedef struct slab_geom { int lpr, cpl; } slab_geom;
@@ -780,7 +782,7 @@ static int slab_path(size_t n_rows, size_t k) {
 /* does a job have the shape of the wide kernel (one without rows has no
  * workgroup there to publish its q / act; the quantiser launch does) */
 static int wide_shape(size_t n_rows, size_t k) {
-    return g.force_path != 1 && n_rows > 0 && k > SLAB_MAX_K && k <= WIDE_MAX_K &&
+    return g.force_path != 1 && n_rows > 0 && n_rows <= UINT32_MAX / 2 && k > SLAB_MAX_K && k <= WIDE_MAX_K &&
            (uint64_t) n_rows * (k / 4) + 32 <= 0xFFFF0000u;
 }
 
@@ -810,7 +812,7 @@ static int reads_written(const sllm_gfx950_gemv_job *a, const sllm_gfx950_gemv_j
  * one reads what another (or itself) writes, one of the two of the wide
  * shape, keep the quantiser launch and the streaming kernel.
  */
-static int wide_allowed(const sllm_gfx950_gemv_job *jobs, size_t n_jobs) {
+static int wide_ordered(const sllm_gfx950_gemv_job *jobs, size_t n_jobs) {
     for (size_t i = 0; i < n_jobs; ++i) {
         if (!wide_shape(jobs[i].n_rows, jobs[i].n)) continue;
         for (size_t j = 0; j < n_jobs; ++j)
@@ -819,7 +821,7 @@ static int wide_allowed(const sllm_gfx950_gemv_job *jobs, size_t n_jobs) {
     return 1;
 }
 
-/* which kernel a job of this shape takes (wide_ok: wide_allowed of its launch's jobs) */
+/* which kernel a job of this shape takes (wide_ok: its launch's wide_target is not 0) */
 enum { PATH_STREAM = 0, PATH_SLAB = 1, PATH_WIDE = 2 };
 static int job_path(size_t n_rows, size_t k, int wide_ok) {
     if (slab_path(n_rows, k)) return PATH_SLAB;
@@ -850,6 +852,50 @@ static uint32_t slab_count(size_t n_rows, size_t k, uint64_t group, uint64_t tar
     return (uint32_t) slabs;
 }
 
+/*
+ * Bytes of packed weights per slab for a batch's jobs of the wide shape, or 0
+ * where the streaming kernel is the better one. A workgroup of the wide
+ * kernel fills a CU, so a second round of them costs as much as the first
+ * (258 workgroups: 80 MB in six tensors of K = 8192 27.8 us, in three, 255
+ * workgroups, 16.4): the slabs are made large enough for at most one workgroup
+ * a CU (now 16.5 for six too). Where that leaves the largest slab far above
+ * the average, where it cannot be done, or past WIDE_KIB a CU, the jobs go to
+ * the streaming kernel. Measured against it and its quantiser launch at K =
+ * 7296 .. 16384, us: one tensor of 136 MiB from f32 x 25 .. 30 against 30 .. 36
+ * (from a quantised row 24 .. 29 against 26 .. 31), of 150 MiB, in two rounds,
+ * 45 .. 55 against 31 .. 38; 171 tensors of 0.64 MB of K = 8192, 1.5 slabs'
+ * worth each and 220 KiB above the average, from their own x 24.9 against
+ * 27.1, from quantised rows 23.1 against 21.6; 512 tensors of 64 rows 17.8
+ * against 18.7 from one x, 15.8 against 15.6 from quantised rows.
+ */
+static uint64_t wide_fit(const sllm_gfx950_gemv_job *jobs, size_t n_jobs) {
+    const uint64_t cu = (uint64_t) (g.cu > 0 ? g.cu : 256);
+    uint64_t bytes = 0, n_wide = 0;
+    int any_x = 0;
+    for (size_t i = 0; i < n_jobs; ++i) {
+        if (!wide_shape(jobs[i].n_rows, jobs[i].n)) continue;
+        any_x |= jobs[i].x != NULL;
+        bytes += (uint64_t) jobs[i].n_rows * (jobs[i].n / 4);
+        if (++n_wide > cu || bytes > cu * WIDE_KIB * 1024u) return 0;
+    }
+    if (n_wide == 0 || g.slab_kib != 0) return slab_default_wide();
+    uint64_t target = (bytes + cu - 1) / cu, wgs, largest;
+    for (;; target += target / 64 + 1) {
+        if (target > bytes) return 0;        /* (tensors of too many rows for one slab's dots) */
+        wgs = largest = 0;
+        for (size_t i = 0; i < n_jobs; ++i) {
+            const size_t n_rows = jobs[i].n_rows, k = jobs[i].n;
+            if (!wide_shape(n_rows, k)) continue;
+            const uint64_t slabs = slab_count(n_rows, k, WIDE_GROUP, target), groups = (n_rows + WIDE_GROUP - 1) / WIDE_GROUP;
+            const uint64_t slab = (groups + slabs - 1) / slabs * WIDE_GROUP * (k / 4);
+            wgs += slabs;
+            if (slab > largest) largest = slab;
+        }
+        if (wgs <= cu) break;
+    }
+    /* a quantiser launch of its own costs the streaming kernel about as much again */
+    return largest * cu <= bytes + cu * WIDE_SLACK_KIB * 1024u * (any_x ? 2u : 1u) ? target : 0;
+}
 
 typedef struct stream_shape {
     int      lpr_idx;
@@ -958,8 +1004,8 @@ static uint64_t pad8(uint64_t v) { return (v + 7u) & ~(uint64_t) 7u; }
  * `kq` (n_jobs entries) the quant list: one row per distinct (x, q) among
  * streaming jobs that carry x, into the job's q / act or into plan scratch
  * (p->scratch_dev, sized by plan_scratch_bytes) shared by every scratch job
- * with the same (x, K). Sets the plan's counts; the descriptors are written
- * by plan_descriptors.
+ * with the same (x, K). p->wide_target is given; sets the plan's counts. The
+ * descriptors are written by plan_descriptors.
  */
 static int plan_layout(const sllm_gfx950_gemv_job *jobs, size_t n_jobs, sllm_gfx950_plan *p,
                        k_quant_job *kq, k_gemv_job *kj, uint8_t *path) {
@@ -971,7 +1017,7 @@ static int plan_layout(const sllm_gfx950_gemv_job *jobs, size_t n_jobs, sllm_gfx
         k_gemv_job *j = &kj[i];
         int st = job_to_kernel(&jobs[i], i, j);
         if (st != SLLM_GFX950_OK) return st;
-        path[i] = (uint8_t) job_path(j->n_rows, j->k, p->wide_ok);
+        path[i] = (uint8_t) job_path(j->n_rows, j->k, p->wide_target != 0);
         if (path[i] == PATH_SLAB) {
             j->variant = (uint32_t) slab_variant_for(j->k);
         } else if (path[i] == PATH_WIDE) {
@@ -1001,20 +1047,14 @@ static int plan_layout(const sllm_gfx950_gemv_job *jobs, size_t n_jobs, sllm_gfx
     }
     /* Slabs of the default size fill the chip with a batch of 35 MB and up;
      * a smaller batch (one FFN set, 13 MB) gets slabs sized so that its
-     * workgroups still cover every CU once. The same for the wide jobs. */
-    uint64_t slab_bytes = 0, wide_bytes = 0;
+     * workgroups still cover every CU once. */
+    uint64_t slab_bytes = 0;
     for (size_t i = 0; i < n_jobs; ++i) {
-        const uint64_t bytes = (uint64_t) kj[i].n_rows * (kj[i].k / 4);
-        if (path[i] == PATH_SLAB) slab_bytes += bytes;
-        if (path[i] == PATH_WIDE) wide_bytes += bytes;
+        if (path[i] == PATH_SLAB) slab_bytes += (uint64_t) kj[i].n_rows * (kj[i].k / 4);
     }
     p->slab_target = slab_default_target();
-    p->wide_target = slab_default_wide();
     if (g.slab_kib == 0 && slab_bytes > 0 && slab_bytes < p->slab_target * (uint64_t) g.cu) {
         p->slab_target = (slab_bytes + (uint64_t) g.cu - 1) / (uint64_t) g.cu;
-    }
-    if (g.slab_kib == 0 && wide_bytes > 0 && wide_bytes < p->wide_target * (uint64_t) g.cu) {
-        p->wide_target = (wide_bytes + (uint64_t) g.cu - 1) / (uint64_t) g.cu;
     }
     for (size_t i = 0; i < n_jobs; ++i) {
         k_gemv_job *j = &kj[i];
@@ -1123,8 +1163,8 @@ int sllm_gfx950_plan_create(const sllm_gfx950_gemv_job *jobs, size_t n_jobs,
         st = fail(SLLM_GFX950_ERR_NOMEM, "plan: host tables");
     }
     if (st == SLLM_GFX950_OK) {
-        p->wide_ok = wide_allowed(jobs, n_jobs);
-        const size_t scratch = plan_scratch_bytes(jobs, n_jobs, p->wide_ok);
+        p->wide_target = wide_ordered(jobs, n_jobs) ? wide_fit(jobs, n_jobs) : 0;
+        const size_t scratch = plan_scratch_bytes(jobs, n_jobs, p->wide_target != 0);
         if (scratch) {
             hipError_t e = hipMalloc(&p->scratch_dev, scratch);
             if (e != hipSuccess) st = hip_fail(e, "plan: activation scratch");
@@ -1220,38 +1260,43 @@ int sllm_gfx950_gemv_batch_noalloc(const sllm_gfx950_gemv_job *jobs, size_t n_jo
                     SLLM_GFX950_NOALLOC_MAX_JOBS);
     }
     const size_t cap = SLLM_GFX950_NOALLOC_SCRATCH_BYTES;
-    const int wide_ok = wide_allowed(jobs, n_jobs);
-    const size_t rows = align256(plan_scratch_bytes(jobs, n_jobs, wide_ok));
-    if (rows > cap) {
-        return fail(SLLM_GFX950_ERR_TOO_LARGE, "gemv_batch_noalloc: %zu bytes of quantised rows, the array holds %zu",
-                    rows, cap);
-    }
-    pthread_mutex_lock(&g_noalloc_mtx);
+    const int ordered = wide_ordered(jobs, n_jobs);
     sllm_gfx950_plan p;
     memset(&p, 0, sizeof p);
     p.scratch_dev = g.noalloc_dev;
-    p.wide_ok = wide_ok;
-    int st = plan_layout(jobs, n_jobs, &p, g_noalloc.quant, g_noalloc.jobs, g_noalloc.path);
-    if (st == SLLM_GFX950_OK) {
-        const size_t qbytes = p.n_quant * sizeof(k_quant_job), jbytes = n_jobs * sizeof(k_gemv_job);
-        const size_t dbytes = ((size_t) p.slab_wg + p.st_wg + p.wide_wg) * sizeof(k_wg_desc);
-        const size_t bytes = qbytes + jbytes + dbytes;
-        if (rows + bytes > cap) {
-            st = fail(SLLM_GFX950_ERR_TOO_LARGE, "gemv_batch_noalloc: %zu bytes of rows and tables, the array holds %zu",
-                      rows + bytes, cap);
-        } else {
-            uint8_t *host = g_noalloc.tables;
-            memcpy(host, g_noalloc.quant, qbytes);
-            memcpy(host + qbytes, g_noalloc.jobs, jbytes);
-            plan_descriptors(&p, g_noalloc.jobs, g_noalloc.path, (k_wg_desc *) (host + qbytes + jbytes));
-            p.tables_dev = (uint8_t *) g.noalloc_dev + rows;
-            hipError_t e = hipMemcpyAsync(p.tables_dev, host, bytes, hipMemcpyHostToDevice, g.stream);
-            if (e != hipSuccess) st = hip_fail(e, "gemv_batch_noalloc: tables");
-            if (st == SLLM_GFX950_OK) st = plan_launch(&p, -1);
-            /* the array and the host staging are free again once the stream drains */
-            e = hipStreamSynchronize(g.stream);
-            if (st == SLLM_GFX950_OK && e != hipSuccess) st = hip_fail(e, "gemv_batch_noalloc: synchronise");
+    p.wide_target = ordered ? wide_fit(jobs, n_jobs) : 0;
+    pthread_mutex_lock(&g_noalloc_mtx);
+    size_t rows, qbytes, jbytes, bytes;
+    int st;
+    for (;;) {
+        rows = align256(plan_scratch_bytes(jobs, n_jobs, p.wide_target != 0));
+        st = rows > cap ? SLLM_GFX950_OK : plan_layout(jobs, n_jobs, &p, g_noalloc.quant, g_noalloc.jobs, g_noalloc.path);
+        if (st != SLLM_GFX950_OK) break;
+        qbytes = p.n_quant * sizeof(k_quant_job);
+        jbytes = n_jobs * sizeof(k_gemv_job);
+        bytes = qbytes + jbytes + ((size_t) p.slab_wg + p.st_wg + p.wide_wg) * sizeof(k_wg_desc);
+        if (rows <= cap && rows + bytes <= cap) break;
+        if (!ordered || p.wide_target != 0) {
+            st = rows > cap ? fail(SLLM_GFX950_ERR_TOO_LARGE, "gemv_batch_noalloc: %zu bytes of quantised rows, the array holds %zu",
+                                   rows, cap)
+                            : fail(SLLM_GFX950_ERR_TOO_LARGE, "gemv_batch_noalloc: %zu bytes of rows and tables, the array holds %zu",
+                                   rows + bytes, cap);
+            break;
         }
+        p.wide_target = slab_default_wide();     /* needs no rows and fewer descriptors than the streaming kernel */
+    }
+    if (st == SLLM_GFX950_OK) {
+        uint8_t *host = g_noalloc.tables;
+        memcpy(host, g_noalloc.quant, qbytes);
+        memcpy(host + qbytes, g_noalloc.jobs, jbytes);
+        plan_descriptors(&p, g_noalloc.jobs, g_noalloc.path, (k_wg_desc *) (host + qbytes + jbytes));
+        p.tables_dev = (uint8_t *) g.noalloc_dev + rows;
+        hipError_t e = hipMemcpyAsync(p.tables_dev, host, bytes, hipMemcpyHostToDevice, g.stream);
+        if (e != hipSuccess) st = hip_fail(e, "gemv_batch_noalloc: tables");
+        if (st == SLLM_GFX950_OK) st = plan_launch(&p, -1);
+        /* the array and the host staging are free again once the stream drains */
+        e = hipStreamSynchronize(g.stream);
+        if (st == SLLM_GFX950_OK && e != hipSuccess) st = hip_fail(e, "gemv_batch_noalloc: synchronise");
     }
     pthread_mutex_unlock(&g_noalloc_mtx);
     return st;
@@ -1268,7 +1313,7 @@ static int single_launch(const sllm_gfx950_gemv_job *j) {
     const k_gemv_job *no_jobs = NULL;
     const k_wg_desc *no_descs = NULL;
     uint32_t zero = 0;
-    const int path = job_path(kj.n_rows, kj.k, wide_allowed(j, 1));
+    const int path = job_path(kj.n_rows, kj.k, wide_shape(kj.n_rows, kj.k) && wide_ordered(j, 1) && wide_fit(j, 1) != 0);
     if (path != PATH_STREAM) {
         const int wide = path == PATH_WIDE;
         kj.variant = wide ? wide_variant(kj.k) : (uint32_t) slab_variant_for(kj.k);

@@ -19,8 +19,8 @@
  *   fakehip_live()               resources held: memory, modules, streams,
  *                                events, graphs
  *   fakehip_calls()              HIP calls made so far
- *   fakehip_launches()           names of the kernels launched since the last
- *                                fakehip_clear, a space behind each
+ *   fakehip_launches()           kernels launched since the last fakehip_clear:
+ *                                name:grid, a space behind each
  */
 #include <hip/hip_runtime_api.h>
 
@@ -184,8 +184,8 @@ hipError_t hipModuleLaunchKernel(hipFunction_t f, unsigned int gx, unsigned int 
     (void) gx; (void) gy; (void) gz; (void) bx; (void) by; (void) bz; (void) lds; (void) s; (void) extra;
     INJECT();
     const char *name = ((const fake_fn *) f)->name;
-    if (g_launches_len + strlen(name) + 2 <= sizeof g_launches) {
-        g_launches_len += (size_t) snprintf(g_launches + g_launches_len, sizeof g_launches - g_launches_len, "%s ", name);
+    if (g_launches_len + strlen(name) + 13 <= sizeof g_launches) {
+        g_launches_len += (size_t) snprintf(g_launches + g_launches_len, sizeof g_launches - g_launches_len, "%s:%u ", name, gx);
     }
     if (strcmp(name, "sllm_k_host_done") == 0) {
         **(uint32_t **) args[0] = *(uint32_t *) args[1];

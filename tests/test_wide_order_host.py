@@ -1,5 +1,7 @@
 """Which kernels a GEMV of 7168 < K <= 16384 takes, on the CPU: the library's C
-sources against the host-memory HIP stand-in, which records the launches.
+sources against the host-memory HIP stand-in (256 CUs), which records the
+launches. The wide kernel is the better one while its workgroups are all
+resident: at most one a CU, of about equal slabs, up to 136 MiB in all.
 Where a call's jobs read what others (or they themselves) write, the wide
 kernel's workgroups would read beside the writes; such a call keeps the
 quantiser launch and the streaming kernel, which order them."""
@@ -12,6 +14,9 @@ from test_failure_injection import _err, fake  # noqa: F401
 
 K, N = 8192, 300
 WIDE, SLAB, STREAM = "sllm_k_gemv_wide", "sllm_k_gemv_slab", "sllm_k_gemv_stream_l8"
+
+
+CU, MAX_BYTES = 256, 256 * 544 * 1024
 
 
 class Mem:
@@ -38,7 +43,14 @@ def lib(fake):  # noqa: F811
 def _launches(L, call):
     L.fakehip_clear()
     assert call() == 0, _err(L)
-    return L.fakehip_launches().decode().split()
+    return [e.split(":")[0] for e in L.fakehip_launches().decode().split()]
+
+
+def _wide_grid(L):
+    """Workgroups of the last call's wide launch."""
+    g = [int(e.split(":")[1]) for e in L.fakehip_launches().decode().split() if e.startswith(WIDE)]
+    assert len(g) == 1
+    return g[0]
 
 
 def _batches(amd, L, jobs):
@@ -118,3 +130,49 @@ def test_job_without_rows_publishes_its_row(amd, lib):
     assert _batches(amd, lib, [amd.GemvJob(w, 0, K, x, q, act, out, None)]) == ["sllm_k_quant_list"]
     assert _batches(amd, lib, [amd.GemvJob(w, 0, K, x, q, act, out, None),
                                amd.GemvJob(w, N, K, x, None, None, out, None)]) == ["sllm_k_quant_list", WIDE]
+
+
+@pytest.mark.parametrize("k", [7296, 8192, 12416, 16384])
+def test_single_tensor_sizes(amd, lib, k):
+    """Up to 136 MiB; nothing is read here, so the weights' extent does not matter."""
+    m = Mem()
+    last = MAX_BYTES // (k // 4)
+    for rows, want in ((1, [WIDE]), (last, [WIDE]), (last + 1, ["sllm_k_quant_act", STREAM])):
+        call = lambda: lib.sllm_gfx950_linear(m.at(400000), rows, k, m.at(0), None, None, 1 << 40)  # noqa: E731,B023
+        assert _launches(lib, call) == want
+        if want == [WIDE]:
+            assert _wide_grid(lib) <= CU
+
+
+@pytest.mark.parametrize("shapes, wide", [
+    ([(1, 8192)] * 256, True), ([(1, 8192)] * 257, False), ([(6510, 8192)] * 6, True), ([(300, 7296)] * 16, True),
+    ([(4096, 14336), (1029, 8192), (16, 7296), (2500, 16384)], True), ([(300, 7296)] * 128, True),
+    ([(314, 8192)] * 171, True), ([(385, 8192)] * 171, False), ([(17408, 16384)] * 2, True), ([(17409, 16384)] * 2, False),
+    ([(20000, 8192)] + [(16, 8192)] * 200, False), ([(0, 8192)] * 300 + [(5, 8192)], True)])
+def test_batches_are_resident_together(amd, lib, shapes, wide):
+    m = Mem()
+    jobs = [amd.GemvJob(m.at(400000), n, k, m.at(0), None, None, 1 << 40, None) for n, k in shapes]
+    arr = (amd.GemvJob * len(jobs))(*jobs)
+    got = _launches(lib, lambda: lib.sllm_gfx950_gemv_batch(arr, len(jobs)))
+    assert [g for g in got if g != "sllm_k_quant_list"] == [WIDE if wide else STREAM]
+    if wide:
+        assert _wide_grid(lib) <= CU
+    # from quantised rows the streaming kernel needs no launch ahead of it
+    jobs = [amd.GemvJob(m.at(400000), n, k, None, m.at(0), None, None, 1 << 40) for n, k in shapes]
+    arr = (amd.GemvJob * len(jobs))(*jobs)
+    if shapes == [(314, 8192)] * 171:
+        wide = False
+    assert _launches(lib, lambda: lib.sllm_gfx950_gemv_batch(arr, len(jobs))) == [WIDE if wide else STREAM]
+
+
+def test_static_array_takes_what_needs_no_rows(amd, lib):
+    """300 rows of 8192 quantised values do not fit the static array; the wide
+    kernel quantises in place. Where the order needs the rows, it is refused."""
+    m = Mem()
+    jobs = [amd.GemvJob(m.at(400000), 16, K, m.at(256 * i), None, None, (1 << 40) + 64 * i, None) for i in range(300)]
+    arr = (amd.GemvJob * 300)(*jobs)
+    assert _launches(lib, lambda: lib.sllm_gfx950_gemv_batch_noalloc(arr, 300)) == [WIDE]
+    assert _launches(lib, lambda: lib.sllm_gfx950_gemv_batch(arr, 300)) == ["sllm_k_quant_list", STREAM]
+    arr[7].out = m.at(512)
+    assert lib.sllm_gfx950_gemv_batch_noalloc(arr, 300) == -36 and "the array holds" in _err(lib)
+    assert _launches(lib, lambda: lib.sllm_gfx950_gemv_batch_noalloc(arr, 20)) == ["sllm_k_quant_list", STREAM]
