@@ -1499,8 +1499,10 @@ int sllm_shim_gemm_qkv_rope(const sllm_gfx950_gemm_job jobs[3], size_t n, const 
     int st = gemm_prepare(jobs, 3, n, q, act, m, &a, &tile, &gx, &gy);
     /* a small chunk takes the 32 x 128 tile for the sake of its store: alone
      * that GEMM is slower than on the tile picked, but by less than the store
-     * kernel's own launch: 2 to 128 tokens of 2B at position 0 take 7 to 11 us
-     * less a layer (63.8 -> 56.8 at 2, 81.8 -> 70.4 at 128). */
+     * kernel's own launch: 2 to 64 tokens take 3 to 6 us less a layer at widths
+     * of 256 to 1024, 7 to 13 at 2048 to 5120 (2B 64.0 -> 57.1 at 2 tokens, 80.9
+     * -> 71.3 at 128) and 13 to 25 at 7168, at position 0 and behind 512; more
+     * tokens than 64 to 128, by the width, have that tile anyway. */
     if (st == SLLM_GFX950_OK && gx != 0 && g.force_gemm_tile == 0 && tile != 9 && n % 256 == 0) {
         st = gemm_prepare_tile(jobs, 3, n, q, act, m, 12, &a, &tile, &gx, &gy);
     }
@@ -1527,9 +1529,16 @@ int sllm_shim_gemm_glu(const uint8_t *w_gate, const uint8_t *w_up, size_t n_rows
     int tile = 0;
     uint64_t gx, gy;
     int st = gemm_prepare(jobs, 2, n, q, act, m, &a, &tile, &gx, &gy);
-    /* as for the QKV store: up to 64 tokens the 32 x 128 tile, for its
-     * silu(gate) * up: 1 to 6 us less a layer (67.7 -> 62.6 at 64 tokens). */
-    if (st == SLLM_GFX950_OK && gx != 0 && g.force_gemm_tile == 0 && tile != 9 && n % 256 == 0) {
+    /* As for the QKV store, the 32 x 128 tile for its silu(gate) * up, where
+     * the picked tile's grid takes more than one round of the CUs (2048 x 5632,
+     * 2560 x 6912, 4096 x 7168, 7168 x 7168 at 33 to 64 tokens: 3 to 6 us less a
+     * layer) or the tensors have at least twice as many rows as columns (0 to
+     * 1.3 us less at 256 x 512 .. 3584 x 7168). Elsewhere the few workgroups
+     * of that tile, each over the whole K, cost more than the launch saved:
+     * 2560 x 1024 1.2 us, 4096 x 4096 1.5, 5120 x 7168 2, 7168 x 2816 7. */
+    const uint64_t cu = (uint64_t) (g.cu > 0 ? g.cu : 256);
+    if (st == SLLM_GFX950_OK && gx != 0 && g.force_gemm_tile == 0 && tile != 9 && n % 256 == 0 &&
+        (gx * gy > cu || n_rows >= 2 * n)) {
         st = gemm_prepare_tile(jobs, 2, n, q, act, m, 12, &a, &tile, &gx, &gy);
     }
     if (st != SLLM_GFX950_OK || gx == 0) return st;
