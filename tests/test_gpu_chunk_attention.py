@@ -56,3 +56,38 @@ def test_row_lengths(amd, orc, dev, base, n, n_ctx):
     g.close()
     o.close()
     _compare(got, want)
+
+
+@pytest.mark.parametrize("n", [33, 150])
+def test_subnormal_values(amd, orc, dev, n):
+    """Values so small that every p * v, and every sum of them, is a subnormal
+    f32; the norm behind the attention, the quantiser and the output projection's
+    scale bring them back to the residual's size, so a matrix instruction that
+    flushed them would change the logits.
+    (The scores have no such test: a product below 2^-126 moves no score, and so no
+    exp, by anything that rounding keeps.)"""
+    base, hd, e = 300, 64, 256
+    model = _model(amd, e, 4, 2, 64, 33)
+    layer = model["layers"][0]
+    rows = 2 * hd
+    at = rows * e // 4
+    layer["wv"][at:at + 4] = np.frombuffer(np.float32(1e-40).tobytes(), np.uint8)      # the tensors' scales
+    layer["wo"][e * e // 4:e * e // 4 + 4] = np.frombuffer(np.float32(1e32).tobytes(), np.uint8)
+    layer["attn_sub_norm"][:] *= np.float32(1e4)
+    toks = np.random.default_rng(n).integers(0, 300, n).astype(np.int32)
+    rng = np.random.default_rng(n + 1)
+    k, v = (rng.standard_normal((1, 2, base, hd)).astype(np.float32) for _ in range(2))
+    v = (v.astype(np.float64) * 2e-39).astype(np.float32)
+    g, o = amd.DeviceDecoder(dev, model, base + n), orc.Decoder(model, base + n)
+    ok, ov = o.caches()
+    ok[:, :, :base], ov[:, :, :base] = k, v
+    g.kv_load(k, v, base)
+    got = g.forward_chunk(toks, base)
+    want = np.stack([o.forward(int(t), base + i) for i, t in enumerate(toks)])
+    flushed = orc.Decoder(model, base + n)               # no values at all: other logits
+    fk, _ = flushed.caches()
+    fk[:, :, :base] = k
+    assert not np.array_equal(flushed.forward(int(toks[0]), base), want[0])
+    for d in (g, o, flushed):
+        d.close()
+    _compare(got, want)

@@ -29,3 +29,24 @@ def test_every_logit(amd, orc, dev, n_embd, n_vocab, n):
     nan = np.isnan(want)
     np.testing.assert_array_equal(np.isnan(got), nan)
     np.testing.assert_array_equal(got.view(np.uint32)[~nan], want.view(np.uint32)[~nan])
+
+
+@pytest.mark.parametrize("norm", [2e-38, 1e-36])
+def test_subnormal_products(amd, orc, dev, norm):
+    """Normalised rows so small that the products with the embedding are
+    subnormal f32, all of them and every sum, or some of them: a matrix
+    instruction that flushed its inputs, products or sums would give other bits."""
+    n_vocab, n = 130, 33
+    model = amd.synth_model(dict(CFG, n_embd=640, n_vocab=n_vocab, n_head=10, n_head_kv=5), 8)
+    model["output_norm"][:] = norm * np.linspace(0.5, 1.5, 640)
+    e = model["tok_embd"].view(np.float16)
+    e[:] = e / np.float16(1024)
+    toks = np.random.default_rng(5).integers(0, n_vocab, n).astype(np.int32)
+    g, o = amd.DeviceDecoder(dev, model, n), orc.Decoder(model, n)
+    got = g.forward_chunk(toks, 0)
+    want = np.stack([o.forward(int(t), i) for i, t in enumerate(toks)])
+    g.close()
+    o.close()
+    low = np.abs(want) < 2.0 ** -126
+    assert np.count_nonzero(want) > 0.9 * want.size and (low.all() if norm == 2e-38 else low.any())
+    np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
