@@ -259,9 +259,9 @@ def test_batch_and_plan_over_a_block_match_oracle(amd, orc, dev):
 
 
 def test_mixed_plan_runs_every_launch_kind(amd, orc, dev):
-    """One plan holding slab jobs (quantising in-kernel and pre-quantised) and
-    K > 7168 jobs that take the streaming kernel, some after a quantiser
-    launch."""
+    """One plan holding slab jobs (quantising in-kernel), a wide job (K up to
+    16384, from a quantised row) and streaming jobs (K above, one of them after a
+    quantiser launch); with the streaming kernel forced, all of them there."""
     specs = [(300, 2560, True), (64, 65536, True), (50, 16384, False), (129, 6912, True), (33, 20480, False)]
     jobs, checks, bufs = [], [], []
     for i, (n_rows, n, fused) in enumerate(specs):

@@ -60,12 +60,13 @@ def _compare(outs, label):
 
 
 def test_noalloc_batch_equals_the_allocating_batch(amd, dev):
-    # slab jobs (K <= 7168) quantising in-kernel, writing q / act, reading a
-    # quantised row; streaming jobs (K > 7168) whose quantised rows go into
-    # the array, or into their own q / act
+    # slab (K <= 7168) and wide jobs (K <= 16384) quantising in-kernel, writing
+    # q / act, reading a quantised row; streaming jobs (larger K) whose quantised
+    # rows go into the array ahead of the tables, or into their own q / act
     first = [(2560, 2560, "x"), (640, 2560, "x"), (6912, 2560, "xq"), (2560, 6912, "q"),
-             (300, 8192, "x"), (129, 16384, "x"), (64, 8192, "xq"), (1000, 1024, "q")]
-    second = [(100, 8192, "x"), (640, 2560, "x")]
+             (300, 8192, "x"), (129, 16384, "x"), (64, 8192, "xq"), (1000, 1024, "q"),
+             (300, 16512, "x"), (129, 20480, "xq"), (64, 65536, "x"), (50, 16512, "q")]
+    second = [(100, 8192, "x"), (640, 2560, "x"), (100, 20480, "x")]
     for label, specs, seed in (("first call", first, 1), ("second, smaller call", second, 2)):
         print(f"[no-alloc] {label}: {len(specs)} jobs", flush=True)
         jobs_a, jobs_b, outs, bufs = _batch(amd, dev, specs, seed)
