@@ -816,7 +816,7 @@ static int wide_ordered(const sllm_gfx950_gemv_job *jobs, size_t n_jobs) {
     for (size_t i = 0; i < n_jobs; ++i) {
         if (!wide_shape(jobs[i].n_rows, jobs[i].n)) continue;
         for (size_t j = 0; j < n_jobs; ++j)
-            if (reads_written(&jobs[i], &jobs[j]) || reads_written(&jobs[j], &jobs[i])) return 0;
+            if (reads_written(&jobs[i], &jobs[j]) || (j != i && reads_written(&jobs[j], &jobs[i]))) return 0;
     }
     return 1;
 }
@@ -880,6 +880,7 @@ static uint64_t wide_fit(const sllm_gfx950_gemv_job *jobs, size_t n_jobs) {
     }
     if (n_wide == 0 || g.slab_kib != 0) return slab_default_wide();
     uint64_t target = (bytes + cu - 1) / cu, wgs, largest;
+    if (n_wide == 1) return target;          /* at most cu slabs, at most a row group above the average */
     for (;; target += target / 64 + 1) {
         if (target > bytes) return 0;        /* (tensors of too many rows for one slab's dots) */
         wgs = largest = 0;
@@ -1313,7 +1314,8 @@ static int single_launch(const sllm_gfx950_gemv_job *j) {
     const k_gemv_job *no_jobs = NULL;
     const k_wg_desc *no_descs = NULL;
     uint32_t zero = 0;
-    const int path = job_path(kj.n_rows, kj.k, wide_shape(kj.n_rows, kj.k) && wide_ordered(j, 1) && wide_fit(j, 1) != 0);
+    const int path = slab_path(kj.n_rows, kj.k) ? PATH_SLAB
+                   : job_path(kj.n_rows, kj.k, wide_ordered(j, 1) && wide_fit(j, 1) != 0);
     if (path != PATH_STREAM) {
         const int wide = path == PATH_WIDE;
         kj.variant = wide ? wide_variant(kj.k) : (uint32_t) slab_variant_for(kj.k);
