@@ -1441,7 +1441,6 @@ static int gemm_prepare_tile(const sllm_gfx950_gemm_job *jobs, size_t n_jobs, si
         else if (m <= 64) tile = gemm_grid(14, jobs, n_jobs, m) * 4 >= cu * 3 ? 14 : 13;
         else if (m <= 256) tile = gemm_grid(12, jobs, n_jobs, m) * 2 >= cu ? 12 : 14;
         else tile = gemm_grid(9, jobs, n_jobs, m) * 4 >= cu * 3 ? 9 : 12;
-        if (n % 256 != 0 && tile == 12 && m > (size_t) 65535 * 32) tile = 2;   /* past its grid: the 64-token tile */
     } else if (tile >= 3 && n % 256 != 0) {
         tile = 2;
     }
@@ -1459,6 +1458,7 @@ static int gemm_prepare_tile(const sllm_gfx950_gemm_job *jobs, size_t n_jobs, si
     }
     a->q = q; a->act = act; a->k = (uint32_t) n; a->m = (uint32_t) m; a->n_jobs = (uint32_t) n_jobs;
     const uint64_t gy = (m + tok_per_wg - 1) / tok_per_wg;
+    if (gx == 0) return SLLM_GFX950_OK;              /* no rows */
     if (gx > INT32_MAX || gy > 65535) return fail(SLLM_GFX950_ERR_TOO_LARGE, "gemm: grid too large");
     *tile_out = tile;
     *gx_out = gx;
