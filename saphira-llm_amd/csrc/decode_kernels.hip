@@ -571,50 +571,46 @@ __device__ __forceinline__ void scores_body(const dec_attn &A) {
 extern "C" __global__ void __launch_bounds__(ATT_THREADS)
 sllm_k_dec_scores(dec_attn A) { scores_body<false>(A); }
 
-// The chunk's scores: workgroup (KV head, 64 positions, TOK tokens), so
-// that a block of cached keys, loaded once into LDS, serves TOK tokens (8;
-// 4 for small chunks, whose grid would otherwise be a few dozen). Thread
-// (h, r) -- wave h is query head h of the KV head, lane r a position --
-// holds TOK dot chains: token by token the q . k of the decode kernel, in
-// order of d, times 1/sqrt(hd), written for the positions at or before each
-// token's own. The queries were roped at their positions by
+// A small chunk's scores: workgroup (KV head, 64 positions, 4 tokens), so
+// that a block of cached keys, loaded once into LDS, serves four tokens (more
+// would leave the grid of a chunk this small at a few dozen workgroups). Thread
+// (h, r) -- wave h is query head h of the KV head, lane r a position -- holds
+// four dot chains: token by token the q . k of the decode kernel, in order of
+// d, times 1/sqrt(hd), written for the positions at or before each token's own.
+// The queries were roped at their positions by the QKV GEMM's epilogue or by
 // sllm_k_chk_kv_store; they are the same for every lane of a wave and come
-// through the scalar unit (8 dimensions of a token per load), so the LDS
+// through the scalar unit (4 dimensions of a token per load), so the LDS
 // serves only the keys.
-typedef float f32x8 __attribute__((ext_vector_type(8)));
+constexpr uint32_t CS_TOK = 4;
 
-template <uint32_t CS_TOK, uint32_t NB = 1>
-__device__ __forceinline__ void chk_scores_body(const dec_attn &A, uint32_t n_tok) {
-    constexpr uint32_t THREADS = ATT_THREADS * NB, LOADS = KT_LOADS / NB;   // NB token blocks per workgroup
+extern "C" __global__ void __launch_bounds__(ATT_THREADS)
+sllm_k_chk_scores4(dec_attn A, uint32_t n_tok) {
     __shared__ __attribute__((aligned(16))) float kt[ATT_POS][KT_STRIDE];
-    const uint32_t kvh = blockIdx.x, s0 = blockIdx.y * ATT_POS, tb0 = blockIdx.z * CS_TOK * NB, tid = threadIdx.x;
-    const uint32_t npast_wg = A.chunk_base + min(tb0 + CS_TOK * NB, n_tok);   // of the workgroup's last token
-    if (s0 >= npast_wg) return;
+    const uint32_t kvh = blockIdx.x, s0 = blockIdx.y * ATT_POS, tb = blockIdx.z * CS_TOK, tid = threadIdx.x;
+    const uint32_t last_tok = min(tb + CS_TOK, n_tok) - 1;
+    const uint32_t npast_max = A.chunk_base + last_tok + 1;
+    if (s0 >= npast_max) return;                     // no position of this block at or before its tokens
     const uint32_t grp = A.n_head / A.n_kv, hd = A.hd, hd4 = hd / 4;
     const float *kc = A.k_cache + (size_t) kvh * A.n_ctx * hd;
 
     // the block's keys (rows past the last token's position re-read a valid row)
-    const uint32_t n_f4 = ATT_POS * hd4, last_cached = npast_wg - 1;
-    f32x4 kv[LOADS];
+    const uint32_t n_f4 = ATT_POS * hd4, last_cached = npast_max - 1;
+    f32x4 kv[KT_LOADS];
 #pragma unroll
-    for (int u = 0; u < (int) LOADS; ++u) {
-        const uint32_t f = min(tid + (uint32_t) u * THREADS, n_f4 - 1);
+    for (int u = 0; u < (int) KT_LOADS; ++u) {
+        const uint32_t f = min(tid + (uint32_t) u * ATT_THREADS, n_f4 - 1);
         kv[u] = *G_CAST(const f32x4, kc + kt_src(f, s0, last_cached, A.n_ctx));
     }
 #pragma unroll
-    for (int u = 0; u < (int) LOADS; ++u) {
-        const uint32_t f = tid + (uint32_t) u * THREADS, r = (f >> 1) % ATT_POS;
-        if (f < n_f4 && s0 + r < npast_wg) *reinterpret_cast<f32x4 *>(&kt[r][kt_col(f)]) = kv[u];
+    for (int u = 0; u < (int) KT_LOADS; ++u) {
+        const uint32_t f = tid + (uint32_t) u * ATT_THREADS, r = (f >> 1) % ATT_POS;
+        if (f < n_f4 && s0 + r < npast_max) *reinterpret_cast<f32x4 *>(&kt[r][kt_col(f)]) = kv[u];
     }
     __syncthreads();
 
-    // wave w: query head w % 4 of the KV head, token block w / 4 of the workgroup's NB
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / ATT_POS), r = tid % ATT_POS, hh = wave % 4u;
-    const uint32_t tb = tb0 + (wave / 4u) * CS_TOK;
-    if (hh >= grp || tb >= n_tok) return;            // uniform; no barriers past this point
-    const uint32_t last_tok = min(tb + CS_TOK, n_tok) - 1;
-    const uint32_t npast_max = A.chunk_base + last_tok + 1;
-    if (s0 >= npast_max) return;                     // no position of this block at or before its tokens
+    // wave w: query head w of the KV head
+    const uint32_t hh = __builtin_amdgcn_readfirstlane(tid / ATT_POS), r = tid % ATT_POS;
+    if (hh >= grp) return;                           // uniform; no barriers past this point
     // the queries are not written during the launch: constant address
     // space, so that their wave-uniform reads are scalar loads
     typedef __attribute__((address_space(4))) const float cfloat;
@@ -670,19 +666,16 @@ __device__ __forceinline__ void chk_scores_body(const dec_attn &A, uint32_t n_to
     }
 }
 
-extern "C" __global__ void __launch_bounds__(ATT_THREADS)
-sllm_k_chk_scores4(dec_attn A, uint32_t n_tok) { chk_scores_body<4>(A, n_tok); }
-
 // The chunk's scores as units of one wave: (KV head, query head, 16 tokens,
 // 64 positions), the same dot chains as above. The products come from the
 // matrix unit: one v_mfma_f32_16x16x1_4b over zeros forms the 16 x 64
 // products of one dimension, each rounded as the reference's multiply (fma
 // with +0; a product of -0 becomes +0, which changes no sum, since no chain
 // ever is -0), and sixteen VALU adds put them on the chains. MFMA and VALU
-// share the SIMD's issue, but a product costs about 1/16 of an instruction
-// instead of one: 1.85 ns per 64 products and sums with two waves per SIMD,
-// against 2.6 at four for a multiply by a scalar and an add, and neither
-// operand passes through the scalar unit. Lane r holds the key of position
+// share the SIMD's issue, but one instruction brings 1024 products: a
+// register-only loop of it and its sixteen adds takes 1.85 ns per 64 products
+// and sums with two waves per SIMD, one of multiplies by a scalar and adds 2.6
+// at four, and neither operand passes through the scalar unit. Lane r holds the key of position
 // s0 + r (one slice of eight dimensions, two 16-byte loads, per eight
 // instructions) and the query of token r % 16; register 4 j + i of lane r is
 // position s0 + 16 j + 4 (r / 16) + i for token r % 16, so the scores are
@@ -690,12 +683,14 @@ sllm_k_chk_scores4(dec_attn A, uint32_t n_tok) { chk_scores_body<4>(A, n_tok); }
 // host pads its LDS so that no second one fits) and takes units cu, cu + G,
 // cu + 2G, ... of the launch's G workgroups, so that every CU has the same
 // number of units to within one, at most one more than the others on each
-// SIMD. Bound by that issue (107 cycles of a SIMD per dimension of a unit,
-// of 32 for the products and 64 for the sums at four cycles each): 512 tokens
-// of 2B over prefixes of 0, 512, 1024 and 1536 positions 23.4, 51.5, 79.8 and
-// 109 us a layer, 85 us on average before.
+// SIMD. Bound by that issue: a dimension of a unit takes a SIMD about 107
+// cycles here and about 70 (29.6 ns) in the register-only loop; how much of the
+// difference is the loads' waits and how much the clock, which drops under f32
+// MFMA, was not measured. 512 tokens of 2B over prefixes of 0, 512, 1024 and
+// 1536 positions 23.4, 51.5, 79.8 and 109 us a layer, 85 us on average before.
 constexpr int CSW_THREADS = 1024;
 constexpr uint32_t CSW_TOK = 16;
+typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ void chk_scores_unit(const dec_attn &A, uint32_t n_tok, uint32_t kvh, uint32_t hh,
@@ -1629,13 +1624,13 @@ sllm_k_chk_kv_store(dec_attn A) {
 //
 // Bound by the FMAs: 256 bytes of operands bring 1024 of them, and with no
 // copies at all 128 tokens x 128256 rows x 2560 take 820 us (two waves per
-// SIMD). This takes 1000 us, 512 tokens 3.8 ms, 16 tokens 155 us (657 MB,
-// 4.2 TB/s); one row per lane and the tokens through the scalar unit took 2.69
-// and 9.7 ms. Measured slower here: the operands straight into registers
-// (1050 us with 16 rows a wave, 1220 with 32), rings of four and six pairs at
-// one workgroup per CU (1340). Workgroups for the same rows and different
-// tokens sit next to each other on one XCD, so the rows come from its L2 after
-// the first.
+// SIMD). This takes 1000 to 1100 us across cards, 512 tokens 4.3 to 4.7 ms, 16
+// tokens 155 us (657 MB, 4.2 TB/s); one row per lane and the tokens through
+// the scalar unit took 2.69 and 9.7 ms. Measured slower here: the operands
+// straight into registers (1050 us with 16 rows a wave, 1220 with 32), rings of
+// four and six pairs at one workgroup per CU (1340). Workgroups for the same
+// rows and different tokens sit next to each other on one XCD, so the rows come
+// from its L2 after the first.
 extern "C" __global__ void __launch_bounds__(CLM_THREADS, 2)
 sllm_k_chk_lm_head(chk_lm L) {
     __shared__ __attribute__((aligned(1024))) uint8_t S[CLM_THREADS / 64 * CLM_RING * CLM_SLOT];
